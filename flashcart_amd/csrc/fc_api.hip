@@ -5,7 +5,7 @@ namespace fc {
 
 int segment_sum(int64_t n_seg, int64_t width, const float* src, const int32_t* perm, const int32_t* ptr, float* dst,
                 hipStream_t s);
-int colsum(int64_t rows, int64_t cols, const float* src, float* dst, hipStream_t s);
+int colsum(int64_t rows, int64_t cols, float* src, float* dst, hipStream_t s);  // src is overwritten
 
 // Runtime mirror of PathList (same order, used for validation and sizes).
 static int count_paths(int l1m, int l2m, int lom, bool sym, int* per_lo) {

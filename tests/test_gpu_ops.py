@@ -586,3 +586,23 @@ def test_shift_vectors_kernel():
     sv = shift_vectors(cg, shifts.to(DEV), idx_i.to(DEV), batch.to(DEV), antisymmetric=True)
     assert sv.grad_fn is not None and torch.equal(sv.detach(), torch_sums(cell, shifts.to(DEV), idx_i.to(DEV),
                                                                           batch.to(DEV)))
+
+
+@pytest.mark.parametrize("n", [1, 15, 33, 64, 65, 1025])
+def test_tp_rows_shared_weight_gradient(n):
+    """The gradient of weights shared by all rows: the column sum over the rows in one pass and in parts,
+    two column tiles (352 columns), against float64. Each term is a sum of at most 25 products; the sum
+    over n rows has at most n / 8 + 16 roundings a chain."""
+    from flashcart_amd import o3
+    C = 32
+    g = torch.Generator(device=DEV).manual_seed(n)
+    tp = o3.TensorProduct(2, 2, 2, C, C, shared_weights=True)
+    a, b = (torch.randn(n, 9 * C, device=DEV, generator=g) for _ in range(2))
+    w = torch.ones(tp.n_total_paths * C, device=DEV, requires_grad=True)
+    out = tp(a, b, w)
+    go = torch.randn(out.shape, device=DEV, generator=g)
+    (gw,) = torch.autograd.grad(out, w, go)
+    w64 = torch.ones(tp.n_total_paths * C, dtype=torch.float64, requires_grad=True)
+    ref = O.tensor_product(a.double().cpu(), b.double().cpu(), w64, None, None, 2, 2, 2, C, C, False, True, False)
+    (want,) = torch.autograd.grad(ref, w64, go.double().cpu())
+    assert_close(gw, want, 0.0, (n / 8 + 41) * 2.0 ** -24 * 25 * n ** 0.5, "shared weight gradient")
