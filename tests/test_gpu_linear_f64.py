@@ -189,3 +189,22 @@ def test_wgrad_entry_points():
                 _close(outs[l], want * (0.75 * scale[l]), f"wgrad n={n} rank {l}")
             io += m * k
             oo += m * fout
+
+
+@pytest.mark.parametrize("n", [1, 31, 63, 64, 65, 1501])
+def test_wgrad_parts(n):
+    """Weight gradients at the row counts where the split into parts of 32 nodes begins and leaves
+    remainders, against float64 on the host: sums of n (2l + 1) products of order one."""
+    lin = lout = 2
+    lay = _layer(lin, lout, 64, 64, [1, 1, 1], 21)
+    x = torch.randn(n, lay.in_dim, device=DEV, dtype=torch.float64)
+    g = torch.randn(n, lay.out_dim, device=DEV, dtype=torch.float64)
+    got = torch.autograd.grad(lay(x), list(lay.weight), g)
+    off = 0
+    for l in range(3):
+        m = (2 * l + 1) * 64
+        xl = x[:, off:off + m].reshape(-1, 64).cpu()
+        gl = g[:, off:off + m].reshape(-1, 64).cpu()
+        want = gl.t() @ xl * lay._scale_list[l]
+        assert_close(got[l], want, 0.0, n * (2 * l + 1) * 2.0 ** -52, f"rank {l}")
+        off += m
