@@ -6,9 +6,9 @@
 // addressed as (node, component), so the packed (n, in_dim) feature rows are read in
 // place; all ranks run in one launch.
 //
-// Two kernels. gemm_pipe_kernel serves every launch whose
-// ranks have K % 32 == 0 and 16-byte aligned rows and need no activation: direct global->LDS
-// loads into a three-stage ring, persistent workgroups, v_mfma_f32_16x16x4f32 blocks.
+// Three kernels. gemm_split_kernel (fc_gemm_split.h) serves every launch whose ranks have K % 32 == 0
+// and 16-byte aligned rows and need no activation. gemm_pairsum_kernel serves the pair sums: direct
+// global->LDS loads into a three-stage ring, persistent workgroups, v_mfma_f32_16x16x4f32 blocks.
 // gemm_kernel serves the rest (activation prologue/epilogue of the dense layers, ragged K):
 // Tiling (gfx950, wave64): 256-thread workgroups, BM x BN output tiles, waves arranged
 // WM x WN, each wave accumulating (BM/WM) x (BN/WN) with v_mfma_f32_32x32x2f32 blocks.
@@ -28,7 +28,7 @@
 // Blocks are ordered N-tile fastest and remapped so that consecutive tiles of one row
 // block land on the same XCD (the hardware deals workgroups round-robin over the 8
 // XCDs), so the A rows are fetched from HBM once and then hit that XCD's L2.
-// fp32 inputs, fp32 accumulation: no reduced-precision operands.
+// float32 inputs and float32 accumulation throughout.
 #include "fc_common.h"
 #include <type_traits>  // std::true_type
 
@@ -373,32 +373,24 @@ __global__ void __launch_bounds__(256) gemm_kernel(GemmBatch gb) {
 }
 
 // ---------------------------------------------------------------------------------------
-// Pipelined GEMM. Operands travel global -> LDS by direct loads (global_load_lds_dwordx4:
-// no register staging, no LDS store phase) into a ring of three stages, so every wave has
-// the next two K steps in flight while it multiplies the current one, with one barrier per
-// K step. Persistent workgroups (two per CU) walk their tiles as one stream of K steps:
-// the first steps of the next tile load during the current tile's epilogue. Used when every
-// rank has K % 32 == 0, 16-byte aligned operand rows and no A prologue (act_bwd) or
-// activation epilogue.
+// Pair-sum GEMM: D = scale (A_lo + A_hi) W^T, where every A row is the sum of two halves of K floats,
+// A[r, 0:K] and A[r, K:2K], or rows a_lo[r] and a_hi[r] of A when the rank gives those index arrays;
+// both halves go to LDS and are added as the MFMA operands are read, so the MFMA work is that of K
+// (the radial output layer's input gradient over edge pairs, whose two edges share the layer's
+// output row). Bound by reading A (9.4 GB at 540,083 pairs and K = 2,176: 1.9-2.1 ms; the split
+// kernel's loads through registers take 2.24 ms there). Operands travel global -> LDS by direct loads
+// (global_load_lds_dwordx4: no register staging, no LDS store phase) into a ring of three stages, so
+// every wave has the next two K steps in flight while it multiplies the current one, with one barrier
+// per K step. Persistent workgroups (two per CU) walk their tiles as one stream of K steps: the first
+// steps of the next tile load during the current tile's epilogue. K % 32 == 0, 16-byte aligned rows.
 //
-// LDS layout per stage: A, and B when k-contiguous (trans_b), as rows of 8 chunks of 4
-// floats (one 32-float K step); chunk c of row r sits at position c ^ ((r / 2) % 8), so the
-// rows read together at one chunk fall in distinct banks (SQ_LDS_BANK_CONFLICT reads 0; the
-// (r % 8)-based swizzle it replaces stalled the LDS ~0.55 of the busy cycles). A k-major B (the input
-// gradient) sits as 32 rows of BN floats; chunk p of row k at p ^ pipe_kswz(k), which puts the
-// rows that the lane groups of one k step read (4 apart) in different parts of the bank row.
-// K-step mapping: MFMA k-pair q (0..3) of quad s4 (0..3) takes k = 8 s4 + 4 h + q in lane
-// half h, in A and B alike, so each lane reads four k values as one 128-bit chunk.
+// LDS layout per stage: rows of 8 chunks of 4 floats (one 32-float K step); chunk c of row r sits at
+// position c ^ ((r / 2) % 8), so the rows read together at one chunk fall in distinct banks
+// (SQ_LDS_BANK_CONFLICT reads 0).
+// K-step mapping: 16x16x4 blocks take k = 16 s + 4 (lane / 16) + q in k-quad q of half s, in A and B
+// alike, so each lane reads four k values as one 128-bit chunk.
 
 __device__ __forceinline__ int pipe_swz(int r) { return (r >> 1) & 7; }
-// k-major B rows: the lane groups reading one k step sit 4 rows apart (2 groups for 32x32x2
-// blocks, 4 for 16x16x4); XOR-ing the chunk index by the group puts each group's 128-byte
-// (32x32) or 64-byte (16x16) column run in its own part of the bank row.
-template <int MI>
-__device__ __forceinline__ int pipe_kswz(int k) {
-  return MI == 32 ? ((k >> 2) & 1) << 3 : ((k >> 2) & 3) << 2;
-}
-
 // One 16-byte direct load per lane into LDS at lds + 16 * lane (lds: byte offset, wave-uniform).
 // Issued as inline assembly so that the compiler does not track it: it would otherwise wait for
 // every outstanding direct load before any LDS read, which defeats the ring. The kernel orders
@@ -412,23 +404,6 @@ __device__ __forceinline__ int pipe_kswz(int k) {
 __device__ __forceinline__ void lds_dma16(const float* src, uint32_t lds_off) {
   asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(lds_off)
                : "memory", "m0");
-}
-
-// The same with a wave-uniform 64-bit base in scalar registers and a 32-bit per-lane byte
-// offset (no per-lane 64-bit address arithmetic per load).
-__device__ __forceinline__ void lds_dma16_s(const float* base, uint32_t voff, uint32_t lds_off) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(base),
-               "s"(lds_off)
-               : "memory", "m0");
-}
-
-// A pointer that is the same in every lane, moved to scalar registers (the asm operands of
-// lds_dma16_s must be scalar).
-__device__ __forceinline__ const float* uniform_ptr(const float* p) {
-  const uint64_t v = (uint64_t)(uintptr_t)p;
-  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);
-  const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
-  return (const float*)(uintptr_t)(((uint64_t)hi << 32) | lo);
 }
 
 // LDS byte address of a __shared__ array (a compile-time constant for a named array)
@@ -451,25 +426,18 @@ struct PipeTile {
   int ri, r0, c0, K;
 };
 
-// PS (pair sum): every A row is the sum of two halves of K floats, A[r, 0:K] and A[r, K:2K], or
-// rows a_lo[r] and a_hi[r] of A when the rank gives those index arrays; both halves go to LDS by
-// direct loads and are added as the MFMA operands are read, so the MFMA work is that of K (the
-// radial output layer's input gradient over edge pairs, whose two edges share the layer's
-// output row).
-template <int BM, int BN, int WM, int WN, int MI, bool KB, bool PS = false>
-__global__ void __launch_bounds__(256, ((PS ? 2 : 1) * BM + BN) * 32 * 4 * 3 <= 80 * 1024 ? 2 : 1) gemm_pipe_kernel(GemmBatch gb) {
-  static_assert(WM * WN == 4, "four waves");
-  static_assert(MI == 32 || MI == 16, "MFMA block: 32x32x2 or 16x16x4");
+constexpr int PAIR_T = 64;  // output tile edge
+
+__global__ void __launch_bounds__(256, 2) gemm_pairsum_kernel(GemmBatch gb) {
+  constexpr int BM = PAIR_T, BN = PAIR_T, WM = 2, WN = 2, MI = 16;
   constexpr int TM = BM / WM, TN = BN / WN;
   constexpr int FM = TM / MI, FN = TN / MI;  // MFMA blocks per wave
-  constexpr int NV = MI == 32 ? 16 : 4;      // accumulator values per lane and block
+  constexpr int NV = 4;                      // accumulator values per lane and block
   typedef float accv __attribute__((ext_vector_type(NV)));
   constexpr int A_DMA = BM * 8 / 256;  // 16-byte chunks per thread and K step
   constexpr int B_DMA = BN * 8 / 256;
-  constexpr int AH = PS ? 2 : 1;       // A halves
+  constexpr int AH = 2;                // A halves
   constexpr int L = AH * A_DMA + B_DMA;  // direct loads per wave and K step
-  static_assert(A_DMA >= 1 && B_DMA >= 1 && L <= 15, "tile shape");
-  constexpr int BQ = BN / 4;           // chunks per k-major B row
   __shared__ __attribute__((aligned(16))) float As0[AH * BM * 32];
   __shared__ __attribute__((aligned(16))) float As1[AH * BM * 32];
   __shared__ __attribute__((aligned(16))) float As2[AH * BM * 32];
@@ -477,7 +445,7 @@ __global__ void __launch_bounds__(256, ((PS ? 2 : 1) * BM + BN) * 32 * 4 * 3 <= 
   __shared__ __attribute__((aligned(16))) float Bs1[BN * 32];
   __shared__ __attribute__((aligned(16))) float Bs2[BN * 32];
 
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6, h = lane >> 5;
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   const int wm = wave / WN, wn = wave % WN;
   const int G = gridDim.x, b = blockIdx.x;
   // Tiles of this workgroup: a contiguous range holding 1/G of the batch's K steps (ranks
@@ -522,83 +490,36 @@ __global__ void __launch_bounds__(256, ((PS ? 2 : 1) * BM + BN) * 32 * 4 * 3 <= 
   };
 
   // ---- producer: direct loads of K steps in tile order
-  // Without pair sums every load of a tile addresses a uniform base (the tile's first A row,
-  // its first B column) plus a 32-bit lane offset fixed for the tile (pipe_ok bounds them);
-  // the pair-sum mode's gathered rows span the whole A, so it keeps 64-bit lane addresses.
-  constexpr bool SADDR = !PS;
   int p_tile = t_first, p_k = 0, n_issued = 0;
   PipeTile pt{0, 0, 0, 32};
-  const float* a_src[SADDR ? 1 : A_DMA];
-  const float* a_src2[PS ? A_DMA : 1];  // second halves
-  const float* b_src[SADDR ? 1 : B_DMA];
-  const float* a_base = nullptr;
-  const float* b_base = nullptr;
-  uint32_t a_off[SADDR ? A_DMA : 1], b_off[SADDR ? B_DMA : 1];  // bytes
+  const float* a_src[A_DMA];
+  const float* a_src2[A_DMA];  // second halves
+  const float* b_src[B_DMA];
   auto p_setup = [&]() {
     if (p_tile >= t_end) return;
     pt = decode(p_tile);
     const GemmRank& g = gb.r[pt.ri];
-    if constexpr (SADDR) {
-      const int n0 = pt.r0 / g.comps, c00 = pt.r0 - n0 * g.comps;
-      const float inv_comps = 1.0f / (float)g.comps;
-      a_base = uniform_ptr(g.A + (int64_t)n0 * g.a_row);
-      b_base = uniform_ptr(KB ? g.B : g.B + (int64_t)pt.c0 * g.K);
-#pragma unroll
-      for (int j = 0; j < A_DMA; ++j) {
-        const int s = (j * 4 + wave) * 64 + lane;
-        const int row = s >> 3, c = (s & 7) ^ pipe_swz(row);
-        const int grow = min(pt.r0 + row, g.M - 1);
-        // node and component counted from node n0: y / comps for y < BM + comps (exact in
-        // float, as in the epilogue)
-        const int y = c00 + (grow - pt.r0);
-        const int dn = (int)(((float)y + 0.5f) * inv_comps), cc = y - dn * g.comps;
-        a_off[j] = 4u * (uint32_t)((int64_t)dn * g.a_row + (int64_t)cc * g.a_comp + 4 * c);
-      }
-#pragma unroll
-      for (int j = 0; j < B_DMA; ++j) {
-        const int s = (j * 4 + wave) * 64 + lane;
-        if constexpr (KB) {
-          const int kk = s / BQ, p = (s % BQ) ^ pipe_kswz<MI>(kk);
-          const int col = min(pt.c0 + 4 * p, g.N - 4);
-          b_off[j] = 4u * (uint32_t)((int64_t)kk * g.N + col);
-        } else {
-          const int col = s >> 3, c = (s & 7) ^ pipe_swz(col);
-          const int gcol = min(pt.c0 + col, g.N - 1);
-          b_off[j] = 4u * (uint32_t)((int64_t)(gcol - pt.c0) * g.K + 4 * c);
-        }
-      }
-      return;
-    }
 #pragma unroll
     for (int j = 0; j < A_DMA; ++j) {
       const int s = (j * 4 + wave) * 64 + lane;
       const int row = s >> 3, c = (s & 7) ^ pipe_swz(row);
       const int grow = min(pt.r0 + row, g.M - 1);
-      if constexpr (PS) {
-        if (g.a_lo) {
-          // Gathered halves. Using these loads waits for every outstanding vector load, the
-          // direct loads of the ring included (once per tile).
-          a_src[j] = g.A + (int64_t)g.a_lo[grow] * g.a_row + 4 * c;
-          a_src2[j] = g.A + (int64_t)g.a_hi[grow] * g.a_row + 4 * c;
-          continue;
-        }
+      if (g.a_lo) {
+        // Gathered halves. Using these loads waits for every outstanding vector load, the
+        // direct loads of the ring included (once per tile).
+        a_src[j] = g.A + (int64_t)g.a_lo[grow] * g.a_row + 4 * c;
+        a_src2[j] = g.A + (int64_t)g.a_hi[grow] * g.a_row + 4 * c;
+        continue;
       }
-      const int n = grow / g.comps, cc = grow - n * g.comps;
-      a_src[j] = g.A + (int64_t)n * g.a_row + (int64_t)cc * g.a_comp + 4 * c;
-      if constexpr (PS) a_src2[j] = a_src[j] + g.K;
+      a_src[j] = g.A + (int64_t)grow * g.a_row + 4 * c;
+      a_src2[j] = a_src[j] + g.K;
     }
 #pragma unroll
     for (int j = 0; j < B_DMA; ++j) {
       const int s = (j * 4 + wave) * 64 + lane;
-      if constexpr (KB) {
-        const int kk = s / BQ, p = (s % BQ) ^ pipe_kswz<MI>(kk);
-        const int col = min(pt.c0 + 4 * p, g.N - 4);
-        b_src[j] = g.B + (int64_t)kk * g.N + col;
-      } else {
-        const int col = s >> 3, c = (s & 7) ^ pipe_swz(col);
-        const int gcol = min(pt.c0 + col, g.N - 1);
-        b_src[j] = g.B + (int64_t)gcol * g.K + 4 * c;
-      }
+      const int col = s >> 3, c = (s & 7) ^ pipe_swz(col);
+      const int gcol = min(pt.c0 + col, g.N - 1);
+      b_src[j] = g.B + (int64_t)gcol * g.K + 4 * c;
     }
   };
   // LDS byte addresses of the stage being filled (as, bs); this wave's 16-byte chunks of a
@@ -606,24 +527,12 @@ __global__ void __launch_bounds__(256, ((PS ? 2 : 1) * BM + BN) * 32 * 4 * 3 <= 
   const uint32_t wave_lds = 1024u * (uint32_t)__builtin_amdgcn_readfirstlane(wave);
   auto p_issue = [&](uint32_t as, uint32_t bs) {
     if (p_tile >= t_end) return;
-    const int64_t bstep = KB ? (int64_t)p_k * gb.r[pt.ri].N : (int64_t)p_k;
-    if constexpr (SADDR) {
-      const float* sa = uniform_ptr(a_base + p_k);
-      const float* sb = uniform_ptr(b_base + bstep);
-#pragma unroll
-      for (int j = 0; j < A_DMA; ++j) lds_dma16_s(sa, a_off[j], as + 4096u * j + wave_lds);
-#pragma unroll
-      for (int j = 0; j < B_DMA; ++j) lds_dma16_s(sb, b_off[j], bs + 4096u * j + wave_lds);
-    } else {
 #pragma unroll
     for (int j = 0; j < A_DMA; ++j) lds_dma16(a_src[j] + p_k, as + 4096u * j + wave_lds);
-    if constexpr (PS) {
 #pragma unroll
-      for (int j = 0; j < A_DMA; ++j) lds_dma16(a_src2[j] + p_k, as + 4u * BM * 32 + 4096u * j + wave_lds);
-    }
+    for (int j = 0; j < A_DMA; ++j) lds_dma16(a_src2[j] + p_k, as + 4u * BM * 32 + 4096u * j + wave_lds);
 #pragma unroll
-    for (int j = 0; j < B_DMA; ++j) lds_dma16(b_src[j] + bstep, bs + 4096u * j + wave_lds);
-    }
+    for (int j = 0; j < B_DMA; ++j) lds_dma16(b_src[j] + p_k, bs + 4096u * j + wave_lds);
     ++n_issued;
     p_k += 32;
     if (p_k >= pt.K) {
@@ -645,38 +554,26 @@ __global__ void __launch_bounds__(256, ((PS ? 2 : 1) * BM + BN) * 32 * 4 * 3 <= 
 #pragma unroll
       for (int v = 0; v < NV; ++v) acc[i][j][v] = 0.f;
 
-  // K mapping inside a 32-float step: 32x32x2 blocks take k = 8 s + 4 (lane / 32) + q in
-  // k-pair q of quad s (4 quads); 16x16x4 blocks take k = 16 s + 4 (lane / 16) + q in k-quad
-  // q of half s (2 halves). Either way a lane reads its four k values as one chunk.
-  constexpr int NS = MI == 32 ? 4 : 2;
-  const int kg = MI == 32 ? h : (lane >> 4);  // lane group along k
+  const int kg = lane >> 4;  // lane group along k
   // FIRST: the tile's first K step, whose first MFMA of each block starts from zero (the
   // accumulators need no clearing between tiles)
   auto compute = [&](const float* as, const float* bs, auto first_c) {
     constexpr bool FIRST = decltype(first_c)::value;
 #pragma unroll
-    for (int s4 = 0; s4 < NS; ++s4) {
+    for (int s4 = 0; s4 < 2; ++s4) {
       float4 a4[FM], b4[FN];
-      const int ch = (MI == 32 ? 2 : 4) * s4 + kg;
+      const int ch = 4 * s4 + kg;
 #pragma unroll
       for (int i = 0; i < FM; ++i) {
         const int row = wm * TM + i * MI + (lane & (MI - 1));
         a4[i] = *reinterpret_cast<const float4*>(as + row * 32 + 4 * (ch ^ pipe_swz(row)));
-        if constexpr (PS) {
-          const float4 hi = *reinterpret_cast<const float4*>(as + BM * 32 + row * 32 + 4 * (ch ^ pipe_swz(row)));
-          a4[i].x += hi.x; a4[i].y += hi.y; a4[i].z += hi.z; a4[i].w += hi.w;
-        }
+        const float4 hi = *reinterpret_cast<const float4*>(as + BM * 32 + row * 32 + 4 * (ch ^ pipe_swz(row)));
+        a4[i].x += hi.x; a4[i].y += hi.y; a4[i].z += hi.z; a4[i].w += hi.w;
       }
 #pragma unroll
       for (int j = 0; j < FN; ++j) {
         const int col = wn * TN + j * MI + (lane & (MI - 1));
-        if constexpr (KB) {
-          const int k = 4 * ch;  // rows k..k+3 share (k / 4) % 2
-          const float* p = bs + k * BN + 4 * ((col >> 2) ^ pipe_kswz<MI>(k)) + (col & 3);
-          b4[j] = make_float4(p[0], p[BN], p[2 * BN], p[3 * BN]);
-        } else {
-          b4[j] = *reinterpret_cast<const float4*>(bs + col * 32 + 4 * (ch ^ pipe_swz(col)));
-        }
+        b4[j] = *reinterpret_cast<const float4*>(bs + col * 32 + 4 * (ch ^ pipe_swz(col)));
       }
 #pragma unroll
       for (int q = 0; q < 4; ++q)
@@ -687,95 +584,31 @@ __global__ void __launch_bounds__(256, ((PS ? 2 : 1) * BM + BN) * 32 * 4 * 3 <= 
             const float a = reinterpret_cast<const float*>(&a4[i])[q];
             const float b = reinterpret_cast<const float*>(&b4[j])[q];
             const accv c = (FIRST && s4 == 0 && q == 0) ? accv{} : acc[i][j];
-            if constexpr (MI == 32) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
-            else acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
           }
     }
   };
 
-  // Residual values are all loaded before the first store: a load into a register that a
-  // pending store still reads would make the compiler wait for every outstanding load,
-  // including the direct loads of the next K steps.
   auto epilogue = [&]() {
     const GemmRank& g = gb.r[ct.ri];
-    const int M = g.M, N = g.N, comps = g.comps;
+    const int M = g.M, N = g.N;
     const float scale = g.scale;
-    // Rows are addressed from the tile's first node (a uniform base) with 32-bit byte
-    // offsets (pipe_ok bounds them), columns j > 0 as immediate offsets: the stores and
-    // residual loads need no per-access 64-bit address arithmetic.
-    const int n0 = ct.r0 / comps, c00 = ct.r0 - n0 * comps;
-    const float inv_comps = 1.0f / (float)comps;
-    gfloat* const Dt = uniform_gptr(g.D + (int64_t)n0 * g.d_row);
-    const bool has_r = g.R != nullptr;
-    const gfloat* const Rt = uniform_gptr(has_r ? g.R + (int64_t)n0 * g.d_row : g.D);
+    // Rows are addressed from the tile's first row (a uniform base) with 32-bit byte offsets (the
+    // caller bounds them), columns j > 0 as immediate offsets.
+    gfloat* const Dt = uniform_gptr(g.D + (int64_t)ct.r0 * g.d_row);
     const int col0 = ct.c0 + wn * TN + (lane & (MI - 1));  // this lane's column in block j = 0
     const bool all_cols = ct.c0 + BN <= N;                  // uniform
-    float bias_v[FN];
-#pragma unroll
-    for (int j = 0; j < FN; ++j) bias_v[j] = (gb.bias && col0 + j * MI < N) ? gb.bias[col0 + j * MI] : 0.f;
-    // block rows of acc value v = 4 vg + q: 8 vg + 4 (lane / 32) + q (32x32), 4 (lane / 16) + q (16x16)
-    uint32_t roff[FM][NV];
-    bool rok[FM][NV];
-#pragma unroll
-    for (int i = 0; i < FM; ++i) {
-#pragma unroll
-      for (int vg = 0; vg < NV / 4; ++vg) {
-        const int rl = wm * TM + i * MI + (MI == 32 ? 8 * vg + 4 * h : 4 * (lane >> 4));
-        // node and component of row r0 + rl, counted from node n0: y / comps for y < BM + comps
-        // (exact in float: (y + 1/2) / comps is at least 1 / (2 comps) from an integer)
-        const int y = c00 + rl;
-        int dn = (int)(((float)y + 0.5f) * inv_comps), c = y - dn * comps;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          rok[i][4 * vg + q] = ct.r0 + rl + q < M;
-          roff[i][4 * vg + q] = 4u * (uint32_t)(dn * (int)g.d_row + c * (int)g.d_comp + col0);
-          if (++c == comps) {
-            c = 0;
-            ++dn;
-          }
-        }
-      }
-    }
-    auto d_at = [&](uint32_t off, int j) { return reinterpret_cast<gfloat*>(reinterpret_cast<gchar*>(Dt) + off) + j * MI; };
-    auto r_at = [&](uint32_t off, int j) {
-      return reinterpret_cast<const gfloat*>(reinterpret_cast<const gchar*>(Rt) + off) + j * MI;
-    };
-#pragma unroll
-    for (int i = 0; i < FM; ++i)
-#pragma unroll
-      for (int j = 0; j < FN; ++j)
-#pragma unroll
-        for (int v = 0; v < NV; ++v) acc[i][j][v] = fmaf(acc[i][j][v], scale, bias_v[j]);
-    if (has_r) {
-      // every residual value is loaded (rows out of range read the tile's first row, columns
-      // out of range nothing) before the first store: a load into a register that a pending
-      // store still reads makes the compiler wait for all outstanding loads, the direct loads
-      // of the next K steps included
-      float rv[FM][NV][FN];
-#pragma unroll
-      for (int i = 0; i < FM; ++i)
-#pragma unroll
-        for (int v = 0; v < NV; ++v)
-#pragma unroll
-          for (int j = 0; j < FN; ++j)
-            rv[i][v][j] = (all_cols || col0 + j * MI < N) ? *r_at(rok[i][v] ? roff[i][v] : 0u, j) : 0.f;
-#pragma unroll
-      for (int i = 0; i < FM; ++i)
-#pragma unroll
-        for (int v = 0; v < NV; ++v)
-#pragma unroll
-          for (int j = 0; j < FN; ++j) acc[i][j][v] += rv[i][v][j];
-    }
-    // nontemporal stores: the output streams to HBM without displacing the operands the next
-    // tiles read from L2 (K = 128 maps 77 -> 81 TFLOP/s alone; 25k-atom step 26.31 -> 26.14 ms)
 #pragma unroll
     for (int i = 0; i < FM; ++i)
 #pragma unroll
       for (int v = 0; v < NV; ++v) {
-        if (!rok[i][v]) continue;
+        const int row = wm * TM + i * MI + 4 * (lane >> 4) + v;  // block row of value v
+        if (ct.r0 + row >= M) continue;
+        const uint32_t off = 4u * (uint32_t)(row * (int)g.d_row + col0);
+        gfloat* const d = reinterpret_cast<gfloat*>(reinterpret_cast<gchar*>(Dt) + off);
 #pragma unroll
         for (int j = 0; j < FN; ++j)
-          if (all_cols || col0 + j * MI < N) __builtin_nontemporal_store(acc[i][j][v], d_at(roff[i][v], j));
+          if (all_cols || col0 + j * MI < N) __builtin_nontemporal_store(acc[i][j][v] * scale, d + j * MI);
       }
   };
 
@@ -825,42 +658,36 @@ static int device_cu_count() {
   return cus[dev];
 }
 
-static bool pipe_ok(const GemmBatch& gb, int n_ranks) {
+// Whether gemm_split_kernel takes the batch.
+static bool split_ok(const GemmBatch& gb, int n_ranks) {
   if (gb.act || gb.act_bwd) return false;
   for (int l = 0; l < n_ranks; ++l) {
     const GemmRank& g = gb.r[l];
     if (g.pre || g.P || g.K < 32 || (g.K & 31) || (g.a_row & 3) || (g.a_comp & 3)) return false;
-    // 32-bit byte offsets of a tile's loads from its first A row / B column (128-row tiles)
-    if ((int64_t)129 * g.a_row + (int64_t)g.comps * g.a_comp + g.K >= (int64_t(1) << 30)) return false;
-    if ((int64_t)128 * g.K >= (int64_t(1) << 30) || (int64_t)32 * g.N + g.N >= (int64_t(1) << 30)) return false;
-    // and of the epilogue's stores from the tile's first output node
+    // 32-bit byte offsets of the epilogue's stores from the tile's first output node (128-row tiles)
     if ((int64_t)129 * g.d_row + (int64_t)g.comps * g.d_comp + g.N >= (int64_t(1) << 30)) return false;
     if (g.d_row > 0x7fffffff || g.d_comp > 0x7fffffff) return false;
-    if (((uintptr_t)g.A & 15) || ((uintptr_t)g.B & 15)) return false;
-    if (!gb.trans_b && (g.N & 3)) return false;
+    if (((uintptr_t)g.A & 15) || (gb.trans_b && ((uintptr_t)g.B & 15))) return false;
   }
   return true;
 }
 
-template <int BM, int BN, int WM, int WN, int MI, bool PS = false>
-int launch_pipe_cfg(GemmBatch gb, int n_ranks, hipStream_t s) {
-  int64_t total = 0;
-  for (int l = 0; l < n_ranks; ++l) {
-    GemmRank& g = gb.r[l];
-    g.tiles_m = (g.M + BM - 1) / BM;
-    g.tiles_n = (g.N + BN - 1) / BN;
-    g.tile_base = (int32_t)total;
-    total += (int64_t)g.tiles_m * g.tiles_n;
-  }
+static int launch_pairsum(GemmBatch gb, hipStream_t s) {
+  GemmRank& g = gb.r[0];
+  if (g.K < 32 || (g.K & 31) || (g.a_row & 3) || ((uintptr_t)g.A & 15) || ((uintptr_t)g.B & 15)) return FC_ERR_SHAPE;
+  if (64 * g.d_row + g.N >= (int64_t(1) << 29)) return FC_ERR_SHAPE;  // the epilogue's byte offsets
+  g.tiles_m = (g.M + PAIR_T - 1) / PAIR_T;
+  g.tiles_n = (g.N + PAIR_T - 1) / PAIR_T;
+  g.tile_base = 0;
+  const int64_t total = (int64_t)g.tiles_m * g.tiles_n;
   if (total == 0) return FC_OK;
   if (total > 0x7fffffff) return FC_ERR_SHAPE;
-  gb.n_ranks = n_ranks;
+  gb.n_ranks = 1;
   gb.total_tiles = (int32_t)total;
   int64_t grid = 2 * (int64_t)device_cu_count();
   if (grid > total) grid = total;
   if (grid >= 8) grid -= grid % 8;
-  if (gb.trans_b) hipLaunchKernelGGL((gemm_pipe_kernel<BM, BN, WM, WN, MI, false, PS>), dim3((unsigned)grid), dim3(256), 0, s, gb);
-  else hipLaunchKernelGGL((gemm_pipe_kernel<BM, BN, WM, WN, MI, true, PS>), dim3((unsigned)grid), dim3(256), 0, s, gb);
+  hipLaunchKernelGGL(gemm_pairsum_kernel, dim3((unsigned)grid), dim3(256), 0, s, gb);
   FC_LAUNCH_CHECK();
   return FC_OK;
 }
@@ -886,6 +713,10 @@ int launch_gemm_cfg(GemmBatch gb, int n_ranks, hipStream_t s) {
   return FC_OK;
 }
 
+}  // namespace fc
+#include "fc_gemm_split.h"
+namespace fc {
+
 int launch_gemm(GemmBatch gb, int n_ranks, hipStream_t s) {
   int max_n = 0;
   int64_t max_m = 0;
@@ -895,30 +726,21 @@ int launch_gemm(GemmBatch gb, int n_ranks, hipStream_t s) {
     if (gb.r[l].M < 0) return FC_ERR_SHAPE;
   }
   if (max_m == 0 || max_n == 0 || n_ranks == 0) return FC_OK;
-  // Measured on the model's shapes (M = n (2l+1) rows, K and N of 128 or paths x 128):
-  // 128 x 64 tiles (waves stacked along M) for the wider input gradients, 64 x 128
-  // (waves side by side along N) for the forward. Both hold four workgroups per CU, whose
-  // prologues and epilogues overlap each other's MFMA work better than two 128 x 128 tiles.
-  // Maps at most 64 wide (the 64-channel models, radial hidden layers) take 64 x 64
-  // tiles: twice the workgroups, so short-K launches fill the chip.
-  // Measured on the model's shapes (MI355X, fp32): the pipelined kernel with 16x16x4 blocks
-  // runs 3-13% faster than the register-staged one; 128 x 64 tiles for maps at most 64 wide
-  // (the radial output layer's input gradient: 112 vs 99 TFLOP/s), 64 x 128 otherwise.
-  // Launches with fewer 128-row tiles than two per CU (the 1,536-atom water box) take 64 x 64
-  // tiles instead, for twice the workgroups.
-  if (gb.pair_sum) {  // forward layout, at most 64 output columns, pipelined kernel only
-    if (!gb.trans_b || max_n > 64 || !pipe_ok(gb, n_ranks)) return FC_ERR_SHAPE;
-    return launch_pipe_cfg<64, 64, 2, 2, 16, true>(gb, n_ranks, s);
+  if (gb.pair_sum) return launch_pairsum(gb, s);
+  if (split_ok(gb, n_ranks)) {
+    // 128-column tiles where they fill the chip (two workgroups per CU) and the map is wider than 64;
+    // 64-column tiles otherwise: twice the workgroups (256 nodes, K of 512 to 896 per rank: 43.6 ->
+    // 30.0 us; at 25,000 nodes the wider tiles are the faster ones, 656 -> 606 us)
+    int64_t tiles = 0;
+    for (int l = 0; l < n_ranks; ++l) tiles += (int64_t)((gb.r[l].M + 127) / 128) * ((gb.r[l].N + 127) / 128);
+    if (max_n > 64 && tiles >= 2 * (int64_t)device_cu_count()) return launch_split_cfg<128>(gb, n_ranks, s);
+    return launch_split_cfg<64>(gb, n_ranks, s);
   }
-  if (pipe_ok(gb, n_ranks)) {
-    if (max_n <= 64) {
-      int64_t tiles128 = 0;
-      for (int l = 0; l < n_ranks; ++l) tiles128 += (gb.r[l].M + 127) / 128;
-      if (tiles128 < 2 * (int64_t)device_cu_count()) return launch_pipe_cfg<64, 64, 2, 2, 16>(gb, n_ranks, s);
-      return launch_pipe_cfg<128, 64, 4, 1, 16>(gb, n_ranks, s);
-    }
-    return launch_pipe_cfg<64, 128, 2, 2, 16>(gb, n_ranks, s);
-  }
+  // Activation prologue or epilogue, ragged K or unaligned rows (M = n (2l+1) rows): 128 x 64 tiles
+  // (waves stacked along M) for the wider input gradients, 64 x 128 (waves side by side along N) for
+  // the forward, 64 x 64 for maps at most 64 wide (twice the workgroups, so short-K launches fill the
+  // chip). All hold four workgroups per CU, whose prologues and epilogues overlap each other's MFMA
+  // work better than two 128 x 128 tiles.
   if (max_n <= 64) return launch_gemm_cfg<64, 64, 2, 2, 1>(gb, n_ranks, s);
   if (!gb.trans_b) return launch_gemm_cfg<128, 64, 4, 1, 1>(gb, n_ranks, s);
   return launch_gemm_cfg<64, 128, 1, 4, 1>(gb, n_ranks, s);

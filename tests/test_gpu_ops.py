@@ -588,6 +588,84 @@ def test_shift_vectors_kernel():
                                                                           batch.to(DEV)))
 
 
+def _map_bound(x, w, k):
+    """Largest error of a float32 map of K terms: every product to 2^-23 (the parts of the split that are
+    left out, below 2^-24, and its own rounding) and K / 16 roundings of the running sum, each at most
+    2^-24 of the sum of magnitudes, with a factor of two for the order inside a matrix instruction."""
+    return (k / 16 + 8) * 2.0 ** -23 * (x.abs() @ w.abs().t())
+
+
+@pytest.mark.parametrize("n,lin,lout,fin,fout,paths", [
+    (1, 0, 0, 32, 4, [1]), (127, 1, 1, 32, 33, [1, 2]), (43, 2, 1, 64, 63, [1, 1, 2]), (129, 0, 0, 96, 65, [1]),
+    (33, 3, 3, 32, 100, [5, 1, 2, 3]), (128, 1, 2, 160, 128, [1, 1]),
+    # enough tiles for 128-column tiles: two column tiles, the second and the last row tile partial
+    (40001, 0, 0, 32, 200, [1]), (8201, 3, 3, 32, 132, [1, 2, 1, 1])])
+def test_linear_split_tiles(n, lin, lout, fin, fout, paths):
+    """The split GEMM at the edges of its tiles (rows, columns, K steps), forward with a residual and input
+    gradient, against float64 with an element-wise bound."""
+    ops = _ops()
+    g = torch.Generator(device=DEV).manual_seed(n + fout)
+    common = min(lin, lout)
+    x = torch.randn(n, sum((2 * l + 1) * fin * paths[l] for l in range(lin + 1)), device=DEV, generator=g)
+    go = torch.randn(n, (lout + 1) ** 2 * fout, device=DEV, generator=g)
+    ws = [torch.randn(fout, fin * paths[l], device=DEV, generator=g) for l in range(common + 1)]
+    scale = [0.25 * (l + 1) for l in range(common + 1)]
+    with torch.no_grad():
+        out = ops.linear_fwd(x, ws, lin, lout, fin, fout, paths, scale, 1.0, go)
+        gx = ops.linear_bwd(go, ws, lin, lout, fin, fout, paths, scale, 1.0)
+    io = oo = 0
+    for l in range(max(lin, lout) + 1):
+        m = 2 * l + 1
+        k = fin * paths[l] if l <= lin else 0
+        gl = go[:, oo:oo + m * fout].reshape(n * m, fout).double() if l <= lout else None
+        if l <= common:
+            xl, w = x[:, io:io + m * k].reshape(n * m, k).double(), ws[l].double()
+            for got, want, bound in (
+                    (out[:, oo:oo + m * fout].reshape(n * m, fout), gl + scale[l] * (xl @ w.t()),
+                     scale[l] * _map_bound(xl, w, k) + 2.0 ** -22 * (gl.abs() + 1)),
+                    (gx[:, io:io + m * k].reshape(n * m, k), scale[l] * (gl @ w),
+                     scale[l] * _map_bound(gl, w.t(), fout))):
+                err = (got.double() - want).abs()
+                assert bool((err <= bound).all()), f"rank {l}: {float((err / bound).max()):.2f} of the bound"
+        elif l <= lout:  # ranks the map does not produce: the residual
+            assert torch.equal(out[:, oo:oo + m * fout], go[:, oo:oo + m * fout])
+        io += m * k
+        oo += m * fout if l <= lout else 0
+
+
+@pytest.mark.parametrize("n,fout", [(70, 40), (40000, 136)])
+def test_linear_split_special_values(n, fout):
+    """Infinities and NaN propagate through the split GEMM as IEEE sums (also where a weight is zero), and
+    operands at both ends of float32's range keep its precision."""
+    ops = _ops()
+    k = 64
+    g = torch.Generator(device=DEV).manual_seed(3)
+    x = torch.randn(n, k, device=DEV, generator=g)
+    w = torch.randn(fout, k, device=DEV, generator=g)
+    w[5, 7] = 0.0
+    x[1, 7] = float("inf")
+    x[33, 9] = float("nan")
+    x[34, 3] = float("-inf")
+    x[40] *= 1e-36
+    x[41] = 0.0
+    x[42] *= 1e36
+    x[43, 0] = 3.4e38  # rounds to infinity in 16 bits
+    w[6] *= 1e-30
+    with torch.no_grad():
+        out = ops.linear_fwd(x, [w], 0, 0, k, fout, [1], [1e-3], 1.0)
+        gx = ops.linear_bwd(out, [w], 0, 0, k, fout, [1], [1.0], 1.0)
+    for a, b, s, got in ((x, w.t(), 1e-3, out), (out, w, 1.0, gx)):
+        want = s * (a.double() @ b.double())
+        assert torch.equal(got.isnan(), want.isnan())
+        finite = want.abs() / s < 3e38  # the unscaled sum overflows float32 past that
+        assert torch.equal(got[want.isinf()], want[want.isinf()].float())
+        rows = torch.isfinite(a).all(1)
+        bound = s * _map_bound(a[rows].double(), b.t().double(), a.shape[1]) + 2.0 ** -126
+        err = (got[rows].double() - want[rows]).abs()
+        assert bool((err <= bound)[finite[rows]].all())
+    assert bool((out[41] == 0).all())
+
+
 @pytest.mark.parametrize("n", [1, 15, 33, 64, 65, 1025])
 def test_tp_rows_shared_weight_gradient(n):
     """The gradient of weights shared by all rows: the column sum over the rows in one pass and in parts,
