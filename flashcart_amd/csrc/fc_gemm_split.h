@@ -23,7 +23,6 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 constexpr float kSplitScale = 0x1p20f, kSplitUnscale = 0x1p-40f;
 
-typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 struct Split8 {

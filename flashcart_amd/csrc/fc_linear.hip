@@ -7,8 +7,8 @@
 // place; all ranks run in one launch.
 //
 // Three kernels. gemm_split_kernel (fc_gemm_split.h) serves every launch whose ranks have K % 32 == 0
-// and 16-byte aligned rows and need no activation. gemm_pairsum_kernel serves the pair sums: direct
-// global->LDS loads into a three-stage ring, persistent workgroups, v_mfma_f32_16x16x4f32 blocks.
+// and 16-byte aligned rows and need no activation. gemm_pairsum_kernel serves the pair sums: direct global->LDS loads into a three-stage ring,
+// persistent workgroups, v_mfma_f32_16x16x4f32 blocks.
 // gemm_kernel serves the rest (activation prologue/epilogue of the dense layers, ragged K):
 // Tiling (gfx950, wave64): 256-thread workgroups, BM x BN output tiles, waves arranged
 // WM x WN, each wave accumulating (BM/WM) x (BN/WN) with v_mfma_f32_32x32x2f32 blocks.
@@ -35,6 +35,7 @@
 namespace fc {
 
 typedef float floatx16 __attribute__((ext_vector_type(16)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr float kSiluScale = 1.6765324703310907f;  // RescaledSiLULayer, src/flashcart/nn/layers.py:23
 
@@ -65,6 +66,11 @@ struct GemmBatch {
 };
 
 __device__ __forceinline__ float sigmoidf_(float x) { return 1.0f / (1.0f + __expf(-x)); }
+
+__device__ __forceinline__ float silu_grad_(float p) {
+  const float s = sigmoidf_(p);
+  return kSiluScale * s * (1.0f + p * (1.0f - s));
+}
 
 constexpr int GEMM_BK = 32;
 constexpr int GEMM_PITCH = GEMM_BK + 4;
@@ -881,149 +887,184 @@ namespace fc {
 
 // ---- Wide output, K = 64: out (n x m) = scale * x (n x 64) @ W^T, W (m x 64), m >> 64 (the
 // radial MLP's output layer, m = paths x channels). Writing the output is as costly as the
-// MFMA work here, so each workgroup keeps its 128 x 64 block of x in LDS and walks the
-// output columns in chunks of 64: the next weight chunk is loaded while the current one
-// is multiplied, and the previous chunk's results are stored in between the MFMAs.
-// MFMA step s (of 32) contracts k = s in lanes 0-31 and k = 32 + s in lanes 32-63, so
-// rows sit in LDS in natural k order (a float4 from global memory is written as is, no
-// register shuffle) and a lane reads four steps with one 128-bit load; the pitch of 68
-// floats (17 x 16 B) keeps those reads conflict-free. Four waves stacked along the rows,
-// 32 x 64 outputs each per chunk.
+// MFMA work here, so each workgroup keeps its 128 x 64 block of x, split into bf16 parts
+// (fc_gemm_split.h), in registers and walks the output columns in chunks of 64 whose weights are
+// split once per workgroup into LDS, double buffered; the next chunk's weights load while the
+// current one is multiplied. Four waves stacked along the rows, 32 x 64 outputs each per chunk.
+// A launch of few row blocks splits the columns over blockIdx.y as well.
+// Measured against float32 matrix instructions before it (m = 2,176): radial MLP of 540,083 rows
+// 1,697 -> 1,299 us (1,377 with stores that are not nontemporal; 4.7 GB written), of 140,000 rows
+// 553 -> 397 us, of 672 rows, where the columns are split, 94 -> 20 us; error against float64
+// 2.5e-7 -> 2.0e-7.
 constexpr int WIDE_BM = 128, WIDE_BN = 64, WIDE_K = 64, WIDE_P = 68;
+constexpr int WIDE_PART = 2 * 4 * 64;  // LDS entries per part of a weight chunk
 
-// Output part shared by the wide kernels: the x block of rows r0 .. r0 + 127 is in As
-// (natural k order, pitch WIDE_P); Bs holds two weight-chunk buffers. Ends with no
-// barrier pending; every thread of the workgroup must call it.
-template <bool GUARD>
-__device__ __forceinline__ void wide_body(const float* As, float (*Bs)[WIDE_BN * WIDE_P], int64_t n, int m,
+// This wave's 32 rows of x: lane (r, h) = (lane % 32, lane / 32) holds k = 16 c + 8 h .. + 7 of row r in
+// chunk c, split and (for sums that come out infinite or NaN) as they are.
+struct WideA {
+  Split8 s[4];
+  f32x4 x[8];
+};
+__device__ __forceinline__ void wide_load_a(const float* row, int h, WideA& a) {
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+#pragma unroll
+    for (int q = 0; q < 2; ++q) a.x[2 * c + q] = *reinterpret_cast<const f32x4*>(row + 16 * c + 8 * h + 4 * q);
+    a.s[c] = split8(a.x[2 * c], a.x[2 * c + 1]);
+  }
+}
+
+// Output part shared by the wide kernels: rows r0 .. r0 + 127, the column chunks of this blockIdx.y.
+// Bs holds two weight chunks: block (column block j, k chunk c) of 64 16-byte entries per part, entry
+// (column % 32 ^ 2 (2 c + h)) + 32 h holding k = 16 c + 8 h .. + 7. Every thread of the workgroup calls it.
+// FULL: every row and column of the block is in range, so the stores are unconditional and the
+// compiler can count them as outstanding where it waits for the next weight chunk.
+template <bool FULL>
+__device__ __forceinline__ void wide_body(const WideA& a, bf16x8 (*Bs)[3 * WIDE_PART], int64_t n, int m,
                                           const float* __restrict__ w, float scale, float* __restrict__ out,
                                           int64_t r0) {
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  auto put4 = [&](float* base, int q, int k4, float4 v) {
-    *reinterpret_cast<float4*>(base + q * WIDE_P + k4) = v;
-  };
-  float4 rb[4];
-  auto load_b = [&](int c0) {  // 64 weight rows x 16 float4, 4 per thread
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6, rl = lane & 31, h = lane >> 5;
+  const int nch_all = (m + WIDE_BN - 1) / WIDE_BN;
+  const int ch0 = (int)((int64_t)nch_all * blockIdx.y / gridDim.y);
+  const int ch1 = (int)((int64_t)nch_all * (blockIdx.y + 1) / gridDim.y);
+  if (ch0 >= ch1) return;  // uniform
+
+  f32x4 br[2][2];
+  auto load_b = [&](int ch) {  // 64 weight rows x 8 groups of 8 k, two per thread
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int e = t + 256 * i, q = e >> 4, k4 = (e & 15) * 4;
-      const int col = c0 + q < m ? c0 + q : m - 1;
-      rb[i] = *reinterpret_cast<const float4*>(w + (int64_t)col * WIDE_K + k4);
+    for (int i = 0; i < 2; ++i) {
+      const int it = t + 256 * i, o = it & 7;
+      const int col = min(ch * WIDE_BN + (it >> 3), m - 1);
+      const float* p = w + (int64_t)col * WIDE_K + 8 * o;
+      br[i][0] = *reinterpret_cast<const f32x4*>(p);
+      br[i][1] = *reinterpret_cast<const f32x4*>(p + 4);
     }
   };
-  // the weight chunk goes to LDS scaled, out = x (W scale)^T (the order of F.linear(x, W * s))
   auto store_b = [&](int buf) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int e = t + 256 * i;
-      put4(Bs[buf], e >> 4, (e & 15) * 4,
-           make_float4(rb[i].x * scale, rb[i].y * scale, rb[i].z * scale, rb[i].w * scale));
-    }
-  };
-  load_b(0);
-  store_b(0);
-  __syncthreads();
-
-  const int half = (lane >> 5) * (WIDE_K / 2);  // k offset of this half-wave
-  const float* as = As + (wave * 32 + (lane & 31)) * WIDE_P + half;
-  const int nch = (m + WIDE_BN - 1) / WIDE_BN;
-  // output rows of this lane: r0 + 32 wave + 8 (v/4) + 4 (lane/32) + v%4
-  const int64_t rl = r0 + wave * 32 + 4 * (lane >> 5);
-  // Unguarded blocks: the element offset of row v (of this lane's 16) from the block's first
-  // element is fixed for the whole block, so a store is a wave-uniform base (the block and the
-  // chunk's column) plus a precomputed 32-bit offset, with no per-store address arithmetic.
-  // (The caller keeps 128 m 4 below 2^31.)
-  uint32_t voff[GUARD ? 1 : 16];  // bytes
-  if constexpr (!GUARD) {
+    for (int i = 0; i < 2; ++i) {
+      const int it = t + 256 * i, o = it & 7, col = it >> 3;
+      const int e = ((col >> 5) * 4 + (o >> 1)) * 64 + ((col & 31) ^ (2 * o)) + 32 * (o & 1);
 #pragma unroll
-    for (int v = 0; v < 16; ++v)
-      voff[v] = (uint32_t)((wave * 32 + 4 * (lane >> 5) + 8 * (v >> 2) + (v & 3)) * m + (lane & 31)) * 4u;
-  }
-  float* const blk = out + r0 * m;
-  // results of output row v (of this lane's 16) and column block j of a chunk at column c0
-  auto store_one = [&](const floatx16 (&res)[2], int c0, int v, int j) {
-    if constexpr (GUARD) {
-      const int64_t row = rl + 8 * (v >> 2) + (v & 3);
-      const int col = c0 + j * 32 + (lane & 31);
-      if (row < n && col < m) out[row * m + col] = res[j][v];
-    } else {
-      *reinterpret_cast<float*>(reinterpret_cast<char*>(blk + c0 + j * 32) + voff[v]) = res[j][v];
+      for (int q = 0; q < 2; ++q) asm volatile("" : "+v"(br[i][q]));
+      const Split8 s = split8(br[i][0], br[i][1]);
+      Bs[buf][e] = s.h;
+      Bs[buf][WIDE_PART + e] = s.m;
+      Bs[buf][2 * WIDE_PART + e] = s.l;
     }
   };
-  // One chunk into `cur`; the previous chunk's results (`prv`, complete by now) are
-  // stored in between this chunk's MFMAs, so the wave keeps the matrix core fed while
-  // its stores issue (two accumulator sets used alternately).
-  auto chunk = [&](int ch, floatx16 (&cur)[2], const floatx16 (&prv)[2], bool have_prev) {
-    const int c0 = ch * WIDE_BN, buf = ch & 1;
-    if (ch + 1 < nch) load_b(c0 + WIDE_BN);
+  // element offset of this lane's 16 output rows from the block's first element (the caller keeps
+  // 128 m 4 below 2^31), so a store is a wave-uniform base plus a 32-bit offset
+  uint32_t voff[16];  // bytes
+#pragma unroll
+  for (int v = 0; v < 16; ++v)
+    voff[v] = (uint32_t)((wave * 32 + 4 * h + 8 * (v >> 2) + (v & 3)) * m + rl) * 4u;
+  gfloat* const blk = uniform_gptr(out + r0 * m);
+  const int64_t row0 = r0 + wave * 32 + 4 * h;
+
+  load_b(ch0);
+  store_b(0);
+  load_b(min(ch0 + 1, ch1 - 1));
+  __syncthreads();
+  int buf = 0;
+  for (int ch = ch0; ch < ch1; ++ch) {
+    floatx16 hi[2], lo[2];
+    auto fetch = [&](int q) {  // group q: k chunk q / 2, column block q % 2
+      const int c = q >> 1, j = q & 1;
+      const bf16x8* p = Bs[buf] + (j * 4 + c) * 64 + (rl ^ (2 * (2 * c + h))) + 32 * h;
+      Split8 f;
+      f.h = p[0];
+      f.m = p[WIDE_PART];
+      f.l = p[2 * WIDE_PART];
+      return f;
+    };
+    Split8 nxt = fetch(0);
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      const int c = q >> 1, j = q & 1;
+      const Split8 b = nxt;
+      if (q + 1 < 8) nxt = fetch(q + 1);
+      __builtin_amdgcn_sched_barrier(0);
+      lo[j] = mfma_bf16(a.s[c].l, b.h, c == 0 ? floatx16{} : lo[j]);
+      hi[j] = mfma_bf16(a.s[c].h, b.h, c == 0 ? floatx16{} : hi[j]);
+      lo[j] = mfma_bf16(a.s[c].h, b.l, lo[j]);
+      lo[j] = mfma_bf16(a.s[c].m, b.m, lo[j]);
+      lo[j] = mfma_bf16(a.s[c].m, b.h, lo[j]);
+      lo[j] = mfma_bf16(a.s[c].h, b.m, lo[j]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    // the next chunk's weights to the other buffer (last read before the barrier that ended the
+    // turn before); loads are issued on every path, so that waits count them exactly
+    store_b(buf ^ 1);
+    __builtin_amdgcn_sched_barrier(0);
+    load_b(min(ch + 2, ch1 - 1));
+    __builtin_amdgcn_sched_barrier(0);
+    const int c0 = ch * WIDE_BN;
+    float probe = 0.f;  // NaN if any sum is infinite or NaN
 #pragma unroll
     for (int j = 0; j < 2; ++j)
 #pragma unroll
-      for (int v = 0; v < 16; ++v) cur[j][v] = 0.f;
-    const float* bs = Bs[buf] + (lane & 31) * WIDE_P + half;
-    // operands of MFMA group s4 + 1 are read from LDS while group s4 multiplies
-    float4 a4n = *reinterpret_cast<const float4*>(as), b4n[2];
-#pragma unroll
-    for (int j = 0; j < 2; ++j) b4n[j] = *reinterpret_cast<const float4*>(bs + j * 32 * WIDE_P);
-#pragma unroll
-    for (int s4 = 0; s4 < 8; ++s4) {  // 32 MFMA steps, four per 128-bit read
-      const float4 a4 = a4n;
-      float4 b4[2] = {b4n[0], b4n[1]};
-      if (s4 + 1 < 8) {
-        const int o = 4 * (s4 + 1);
-        a4n = *reinterpret_cast<const float4*>(as + o);
-#pragma unroll
-        for (int j = 0; j < 2; ++j) b4n[j] = *reinterpret_cast<const float4*>(bs + j * 32 * WIDE_P + o);
+      for (int v = 0; v < 16; ++v) {
+        hi[j][v] = (hi[j][v] + lo[j][v]) * kSplitUnscale;
+        probe = fmaf(hi[j][v], 0.f, probe);
       }
-      __builtin_amdgcn_sched_barrier(0);  // keep those reads ahead of this group's MFMAs
+    if (__any(probe != probe)) {  // again in plain float32
 #pragma unroll
-      for (int q = 0; q < 4; ++q)
+      for (int j = 0; j < 2; ++j) {
+        const float* p = w + (int64_t)min(c0 + 32 * j + rl, m - 1) * WIDE_K + 8 * h;
+        hi[j] = floatx16{};
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          cur[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(reinterpret_cast<const float*>(&a4)[q],
-                                                        reinterpret_cast<const float*>(&b4[j])[q], cur[j], 0, 0, 0);
-          if (have_prev && (q & 1) == 0) store_one(prv, c0 - WIDE_BN, 2 * s4 + (q >> 1), j);
+        for (int q = 0; q < 8; ++q) {
+          const f32x4 bv = *reinterpret_cast<const f32x4*>(p + 16 * (q >> 1) + 4 * (q & 1));
+#pragma unroll
+          for (int i = 0; i < 4; ++i) hi[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a.x[q][i], bv[i], hi[j], 0, 0, 0);
         }
+      }
     }
-    if (ch + 1 < nch) {
-      store_b(buf ^ 1);  // the other buffer was last read in the previous chunk
-      __syncthreads();
+    gfloat* const base = blk + c0;
+    if constexpr (FULL) {
+#pragma unroll
+      for (int v = 0; v < 16; ++v)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          __builtin_nontemporal_store(hi[j][v] * scale,
+                                      reinterpret_cast<gfloat*>(reinterpret_cast<gchar*>(base) + voff[v]) + j * 32);
+    } else {
+#pragma unroll
+      for (int v = 0; v < 16; ++v)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          if (row0 + 8 * (v >> 2) + (v & 3) < n && c0 + j * 32 + rl < m)
+            *(reinterpret_cast<gfloat*>(reinterpret_cast<gchar*>(base) + voff[v]) + j * 32) = hi[j][v] * scale;
     }
-  };
-  floatx16 r0acc[2], r1acc[2];
-  for (int ch = 0; ch < nch; ch += 2) {
-    chunk(ch, r0acc, r1acc, ch > 0);
-    if (ch + 1 < nch) chunk(ch + 1, r1acc, r0acc, true);
+    __syncthreads();
+    buf ^= 1;
   }
-  const int last = nch - 1;
-#pragma unroll
-  for (int v = 0; v < 16; ++v)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) store_one((last & 1) ? r1acc : r0acc, last * WIDE_BN, v, j);
 }
 
-// GUARD = false: every row and column of the block is in range (m a multiple of 64), so
-// the stores are unconditional and the compiler can count them as outstanding rather
-// than wait for them before the next weight chunk is written to LDS. The last, partial
-// row block runs as a separate GUARD = true launch. (The radial MLP forward instead takes
-// the guarded body for its partial block inside the one launch; there it costs no spills.)
-template <bool GUARD>
+__device__ __forceinline__ void wide_out(const WideA& a, bf16x8 (*Bs)[3 * WIDE_PART], int64_t n, int m,
+                                         const float* __restrict__ w, float scale, float* __restrict__ out, int64_t r0) {
+  if (r0 + WIDE_BM <= n && m % WIDE_BN == 0) wide_body<true>(a, Bs, n, m, w, scale, out, r0);
+  else wide_body<false>(a, Bs, n, m, w, scale, out, r0);
+}
+
+// Row blocks x column parts of the wide kernels: two workgroups per CU where the columns allow it.
+static dim3 wide_grid(int64_t blocks, int m) {
+  const int64_t chunks = (m + WIDE_BN - 1) / WIDE_BN, want = 2 * (int64_t)device_cu_count();
+  int64_t parts = blocks > 0 ? (want + blocks - 1) / blocks : 1;
+  if (parts > chunks) parts = chunks;
+  return dim3((unsigned)blocks, (unsigned)parts);
+}
+
 __global__ void __launch_bounds__(256, 2) gemm_wide_kernel(int64_t n, int m, const float* __restrict__ x,
                                                             const float* __restrict__ w, float scale,
-                                                            float* __restrict__ out, int64_t first_block) {
-  __shared__ __attribute__((aligned(16))) float As[WIDE_BM * WIDE_P];
-  __shared__ __attribute__((aligned(16))) float Bs[2][WIDE_BN * WIDE_P];
+                                                            float* __restrict__ out) {
+  __shared__ bf16x8 Bs[2][3 * WIDE_PART];
   const int t = threadIdx.x;
-  const int64_t r0 = (first_block + blockIdx.x) * WIDE_BM;
-  // x block: 128 rows x 16 float4, 8 per thread; rows past n read row n-1 (never stored)
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int e = t + 256 * i, q = e >> 4, k4 = (e & 15) * 4;
-    int64_t row = r0 + q;
-    row = row < n ? row : n - 1;
-    *reinterpret_cast<float4*>(As + q * WIDE_P + k4) = *reinterpret_cast<const float4*>(x + row * WIDE_K + k4);
-  }
-  wide_body<GUARD>(As, Bs, n, m, w, scale, out, r0);
+  const int64_t r0 = (int64_t)blockIdx.x * WIDE_BM, row = r0 + 32 * (t >> 6) + (t & 31);
+  WideA a;
+  wide_load_a(x + (row < n ? row : n - 1) * WIDE_K, (t >> 5) & 1, a);  // rows past n are not stored
+  wide_out(a, Bs, n, m, w, scale, out, r0);
 }
 
 // ---- Radial MLP with two hidden layers of 64 (reference InteractionLayer.radial_mlp,
@@ -1184,16 +1225,27 @@ __device__ __forceinline__ void acc_to_rows(const floatx16 (&acc)[2], float* As,
 
 // HIDDEN: stop after the second hidden layer and write its activation h2 (n x 64) instead of
 // the output layer (the first interaction layer's species density takes h2 itself).
-template <bool GUARD, bool HIDDEN = false>
+template <bool HIDDEN>
 __global__ void __launch_bounds__(256, 2) radial_mlp_fwd_kernel(int64_t n, int n_in, const float* __restrict__ x,
                                                                  const float* __restrict__ w0, float s0,
                                                                  const float* __restrict__ w1, float s1, int m,
                                                                  const float* __restrict__ w2, float s2,
-                                                                 float* __restrict__ out, int64_t first_block) {
-  __shared__ __attribute__((aligned(16))) float As[WIDE_BM * WIDE_P];
-  __shared__ __attribute__((aligned(16))) float Bs[2][WIDE_BN * WIDE_P];
+                                                                 float* __restrict__ out) {
+  // the hidden layers' operands, then the output layer's weight chunks
+  union Lds {
+    struct {
+      float As[WIDE_BM * WIDE_P];
+      float Bs[2][WIDE_BN * WIDE_P];
+    } f;
+    bf16x8 wide[2][3 * WIDE_PART];
+    __device__ Lds() {}
+  };
+  __shared__ __attribute__((aligned(16))) char raw[sizeof(Lds)];
+  Lds& lds = *reinterpret_cast<Lds*>(raw);
+  float* const As = lds.f.As;
+  auto Bs = lds.f.Bs;
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  const int64_t r0 = (first_block + blockIdx.x) * WIDE_BM;
+  const int64_t r0 = (int64_t)blockIdx.x * WIDE_BM;
   mlp_stage_x(As, n, n_in, x, r0);
   mlp_stage_weights(Bs[0], Bs[1], n_in, w0, w1);
   __syncthreads();
@@ -1216,11 +1268,13 @@ __global__ void __launch_bounds__(256, 2) radial_mlp_fwd_kernel(int64_t n, int n
       }
     return;
   }
-  __syncthreads();  // reads of h1 and of both weight buffers done before they are overwritten
+  __syncthreads();  // reads of h1 done before it is overwritten
   acc_to_rows(acc, As, wave, lane, [&](float a) { return silu_r(a * s1); });
   __syncthreads();
-  if (GUARD || r0 + WIDE_BM > n) wide_body<true>(As, Bs, n, m, w2, s2, out, r0);
-  else wide_body<false>(As, Bs, n, m, w2, s2, out, r0);
+  WideA a;
+  wide_load_a(As + (wave * 32 + (lane & 31)) * WIDE_P, lane >> 5, a);
+  __syncthreads();  // reads of h2 and of both weight matrices done before the weight chunks overwrite them
+  wide_out(a, lds.wide, n, m, w2, s2, out, r0);
 }
 
 // Input gradient of the two hidden layers: given gh2 = dL/dh2 (n, 64),
@@ -1324,20 +1378,13 @@ extern "C" int fc_dense_fwd(int64_t n, int32_t k, int32_t m, const float* x, con
   if (n == 0) return FC_OK;
   if (!x || !w || !out) return FC_ERR_NULL;
   if (n > 0x7fffffff) return FC_ERR_SHAPE;
-  if (k == WIDE_K && m >= 4 * WIDE_BN && !bias && act == 0 && ((uintptr_t)x & 15) == 0 && ((uintptr_t)w & 15) == 0) {
+  // (output rows are addressed with 32-bit byte offsets in a block: 128 m 4 < 2^31)
+  if (k == WIDE_K && m >= 4 * WIDE_BN && m < (1 << 22) && !bias && act == 0 && ((uintptr_t)x & 15) == 0 &&
+      ((uintptr_t)w & 15) == 0) {
     const int64_t blocks = (n + WIDE_BM - 1) / WIDE_BM;
-    // unguarded blocks address their 128 rows with 32-bit byte offsets: 128 m 4 < 2^31
-    const int64_t full = (m % WIDE_BN == 0 && (int64_t)m < (int64_t(1) << 22)) ? n / WIDE_BM : 0;
-    if (full > 0) {
-      hipLaunchKernelGGL(gemm_wide_kernel<false>, dim3((unsigned)full), dim3(256), 0, (hipStream_t)stream, n, m, x,
-                         w, scale, out, (int64_t)0);
-      FC_LAUNCH_CHECK();
-    }
-    if (blocks > full) {
-      hipLaunchKernelGGL(gemm_wide_kernel<true>, dim3((unsigned)(blocks - full)), dim3(256), 0, (hipStream_t)stream,
-                         n, m, x, w, scale, out, full);
-      FC_LAUNCH_CHECK();
-    }
+    hipLaunchKernelGGL(gemm_wide_kernel, wide_grid(blocks, m), dim3(256), 0, (hipStream_t)stream, n, m, x, w, scale,
+                       out);
+    FC_LAUNCH_CHECK();
     return FC_OK;
   }
   GemmBatch gb{};
@@ -1381,14 +1428,9 @@ extern "C" int fc_radial_mlp_fwd(int64_t n, int32_t n_in, const float* x, const 
   if (((uintptr_t)w2 & 15) != 0) return FC_ERR_SHAPE;  // weight chunks load as float4
   const int64_t blocks = (n + WIDE_BM - 1) / WIDE_BM;
   if (blocks > 0x7fffffff) return FC_ERR_SHAPE;
-  // one launch (the partial last row block is guarded inside it); unguarded blocks address their
-  // 128 rows with 32-bit byte offsets: 128 m 4 < 2^31
-  if (m % WIDE_BN == 0 && (int64_t)m < (int64_t(1) << 22))
-    hipLaunchKernelGGL(radial_mlp_fwd_kernel<false>, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, n,
-                       (int)n_in, x, w0, s0, w1, s1, (int)m, w2, s2, out, (int64_t)0);
-  else
-    hipLaunchKernelGGL(radial_mlp_fwd_kernel<true>, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, n,
-                       (int)n_in, x, w0, s0, w1, s1, (int)m, w2, s2, out, (int64_t)0);
+  if (m >= (1 << 22)) return FC_ERR_SHAPE;  // 32-bit byte offsets inside a block: 128 m 4 < 2^31
+  hipLaunchKernelGGL(radial_mlp_fwd_kernel<false>, wide_grid(blocks, m), dim3(256), 0, (hipStream_t)stream, n,
+                     (int)n_in, x, w0, s0, w1, s1, (int)m, w2, s2, out);
   FC_LAUNCH_CHECK();
   return FC_OK;
 }
@@ -1400,8 +1442,8 @@ extern "C" int fc_radial_mlp_hidden_fwd(int64_t n, int32_t n_in, const float* x,
   if (!x || !w0 || !w1 || !h2) return FC_ERR_NULL;
   const int64_t blocks = (n + WIDE_BM - 1) / WIDE_BM;
   if (blocks > 0x7fffffff) return FC_ERR_SHAPE;
-  hipLaunchKernelGGL((radial_mlp_fwd_kernel<true, true>), dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, n,
-                     (int)n_in, x, w0, s0, w1, s1, 64, (const float*)nullptr, 1.0f, h2, (int64_t)0);
+  hipLaunchKernelGGL(radial_mlp_fwd_kernel<true>, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, n,
+                     (int)n_in, x, w0, s0, w1, s1, 64, (const float*)nullptr, 1.0f, h2);
   FC_LAUNCH_CHECK();
   return FC_OK;
 }
@@ -1564,11 +1606,6 @@ struct WgradBatch {
   int64_t total_elems;
   float* part;
 };
-
-__device__ __forceinline__ float silu_grad_(float p) {
-  const float s = sigmoidf_(p);
-  return kSiluScale * s * (1.0f + p * (1.0f - s));
-}
 
 // Four consecutive floats of row r starting at column col (zero outside the row range and
 // past the last column), times act'(pre) when P is given.

@@ -684,3 +684,42 @@ def test_tp_rows_shared_weight_gradient(n):
     ref = O.tensor_product(a.double().cpu(), b.double().cpu(), w64, None, None, 2, 2, 2, C, C, False, True, False)
     (want,) = torch.autograd.grad(ref, w64, go.double().cpu())
     assert_close(gw, want, 0.0, (n / 8 + 41) * 2.0 ** -24 * 25 * n ** 0.5, "shared weight gradient")
+
+
+@pytest.mark.parametrize("n,k,m,act", [(20001, 64, 64, 1), (9001, 256, 64, 1), (70, 20, 18, 1), (1, 64, 64, 1),
+                                       # the wide output: columns in parts and whole, partial rows and chunks
+                                       (1, 64, 256, 0), (129, 64, 2180, 0), (65665, 64, 260, 0)])
+def test_dense_tiles(n, k, m, act):
+    """Dense layers in each kernel's range, pre-activation, output and input gradient (with the SiLU derivative
+    on the way in) against float64; a row that holds an infinity gives what IEEE sums give. The SiLU and its
+    derivative change a value by at most twice its error; exp adds 2^-20 of the value."""
+    ops = _ops()
+    g = torch.Generator(device=DEV).manual_seed(n + m)
+    x, w, go = (torch.randn(*s, device=DEV, generator=g) for s in ((n, k), (m, k), (n, m)))
+    if n > 1:
+        x[n - 1, 3] = float("inf")
+    with torch.no_grad():
+        out, pre = ops.dense_fwd(x, w, None, 0.125, act)
+        gx = ops.dense_bwd(go, pre, w, 0.125, act)
+    want_pre = 0.125 * (x.double() @ w.double().t())
+    bound = 0.125 * _map_bound(x.double(), w.double(), k)
+    rows = slice(0, max(1, n - 1))
+    if act:
+        z = want_pre.clone().requires_grad_(True)
+        with torch.enable_grad():
+            want = O.silu(z)
+            (dz,) = torch.autograd.grad(want.sum(), z)
+        assert bool(((pre.double() - want_pre).abs() <= bound)[rows].all())
+        assert bool(((out.double() - want).abs() <= 2 * bound + 2.0 ** -20 * want.abs())[rows].all())
+        a = go.double() * dz
+        slack = 2 * go.double().abs() * bound + 2.0 ** -20 * go.double().abs()
+    else:
+        assert bool(((out.double() - want_pre).abs() <= bound)[rows].all())
+        a, slack = go.double(), 0.0 * go.double()
+    if n > 1:
+        last = (pre if act else out)[n - 1]
+        assert torch.equal(last.isnan(), want_pre[n - 1].isnan())
+        assert torch.equal(last.isinf(), want_pre[n - 1].isinf())
+    want_gx = 0.125 * (a @ w.double())
+    gx_bound = 0.125 * _map_bound(a, w.double().t(), m) + 0.125 * (slack @ w.double().abs())
+    assert bool(((gx.double() - want_gx).abs() <= gx_bound)[rows].all())
