@@ -6,8 +6,9 @@
 // addressed as (node, component), so the packed (n, in_dim) feature rows are read in
 // place; all ranks run in one launch.
 //
-// Three kernels. gemm_split_kernel (fc_gemm_split.h) serves every launch whose ranks have K % 32 == 0
-// and 16-byte aligned rows and need no activation. gemm_pairsum_kernel serves the pair sums: direct global->LDS loads into a three-stage ring,
+// Four kernels. gemm_small_kernel serves launches of little work (small_ok). gemm_split_kernel
+// (fc_gemm_split.h) serves every other launch whose ranks have K % 32 == 0 and 16-byte aligned rows and need
+// no activation. gemm_pairsum_kernel serves the pair sums: direct global->LDS loads into a three-stage ring,
 // persistent workgroups, v_mfma_f32_16x16x4f32 blocks.
 // gemm_kernel serves the rest (activation prologue/epilogue of the dense layers, ragged K):
 // Tiling (gfx950, wave64): 256-thread workgroups, BM x BN output tiles, waves arranged
@@ -698,6 +699,149 @@ static int launch_pairsum(GemmBatch gb, hipStream_t s) {
   return FC_OK;
 }
 
+// GEMM of few rows (a unit cell, a molecule): the tiles above would leave most of the chip idle and
+// walk K serially. Here a workgroup owns a 16 x 16 output block and its four waves each take a quarter of K,
+// straight from global memory into v_mfma_f32_16x16x4f32 operands (lane (r, q) = (lane % 16, lane / 16)
+// loads k = 16 c + 4 q .. + 3 of A row r and of output column r), U chunks of 16 k in flight at once,
+// no LDS until the four partial blocks are added in wave order. Takes every batch whose rows of 4 k are
+// aligned, with the dense layers' activation prologue and epilogue; PS as in gemm_pairsum_kernel.
+template <bool KB, bool PS, int U>
+__global__ void __launch_bounds__(256) gemm_small_kernel(GemmBatch gb) {
+  __shared__ float red[4][16][17];
+  const int b = blockIdx.x;
+  int ri = 0;
+#pragma unroll
+  for (int q = 1; q < FC_MAX_RANKS; ++q)
+    if (q < gb.n_ranks && b >= gb.r[q].tile_base) ri = q;
+  ri = __builtin_amdgcn_readfirstlane(ri);
+  const GemmRank& g = gb.r[ri];
+  const int local = b - g.tile_base;
+  const int r0 = (local / g.tiles_n) * 16, c0 = (local % g.tiles_n) * 16;
+  const int K = g.K, N = g.N, M = g.M;
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6, r = lane & 15, kq = 4 * (lane >> 4);
+  const int row = min(r0 + r, M - 1), col = min(c0 + r, N - 1);
+  const int n = row / g.comps;
+  const int64_t a_off = (int64_t)n * g.a_row + (int64_t)(row - n * g.comps) * g.a_comp;
+  const float *ap, *ap2 = nullptr;
+  const float* const pp = gb.act_bwd && g.P ? g.P + a_off : nullptr;
+  if (PS && g.a_lo) {
+    ap = g.A + (int64_t)g.a_lo[row] * g.a_row;
+    ap2 = g.A + (int64_t)g.a_hi[row] * g.a_row;
+  } else {
+    ap = g.A + a_off;
+    if (PS) ap2 = ap + K;
+  }
+  const float* const bp = KB ? g.B + col : g.B + (int64_t)col * K;
+  // chunks of 16 k: wave w takes the w-th quarter of them
+  const int chunks = (K + 15) >> 4, per = (chunks + 3) >> 2;
+  const int ch0 = wave * per, ch1 = min(ch0 + per, chunks);
+  // one accumulator per chunk in flight, added pairwise at the end: shorter chains of roundings, and the
+  // matrix instructions of the chunks do not wait for each other
+  f32x4 acc[U];
+#pragma unroll
+  for (int i = 0; i < U; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int ch = ch0; ch < ch1; ch += U) {
+    f32x4 av[U], bv[U];
+#pragma unroll
+    for (int i = 0; i < U; ++i) {
+      // a group of 4 k past the end reads the row's first (every K takes 4 or more) and counts as zero
+      const int k = 16 * (ch + i) + kq;
+      const bool ok = ch + i < ch1 && k < K;
+      const int ks = ok ? k : 0;
+      av[i] = *reinterpret_cast<const f32x4*>(ap + ks);
+      if constexpr (PS) av[i] += *reinterpret_cast<const f32x4*>(ap2 + ks);
+      if (pp) {
+        const f32x4 p = *reinterpret_cast<const f32x4*>(pp + ks);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) av[i][q] *= silu_grad_(p[q]);
+      }
+      if constexpr (KB) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) bv[i][q] = bp[(int64_t)(ks + q) * N];
+      } else {
+        bv[i] = *reinterpret_cast<const f32x4*>(bp + ks);
+      }
+      if (!ok) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) av[i][q] = bv[i][q] = 0.f;
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int i = 0; i < U; ++i)
+        acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[i][q], bv[i][q], acc[i], 0, 0, 0);
+  }
+#pragma unroll
+  for (int w = 1; w < U; w *= 2)
+#pragma unroll
+    for (int i = 0; i + w < U; i += 2 * w) acc[i] += acc[i + w];
+#pragma unroll
+  for (int v = 0; v < 4; ++v) red[wave][4 * (lane >> 4) + v][r] = acc[0][v];
+  __syncthreads();
+  const int orow = r0 + (t >> 4), ocol = c0 + (t & 15);
+  if (orow >= M || ocol >= N) return;
+  float x = (red[0][t >> 4][t & 15] + red[1][t >> 4][t & 15]) + (red[2][t >> 4][t & 15] + red[3][t >> 4][t & 15]);
+  x = fmaf(x, g.scale, gb.bias ? gb.bias[ocol] : 0.f);
+  const int on = orow / g.comps;
+  const int64_t off = (int64_t)on * g.d_row + (int64_t)(orow - on * g.comps) * g.d_comp + ocol;
+  if (g.pre) g.pre[off] = x;
+  if (gb.act) x = kSiluScale * x * sigmoidf_(x);
+  if (g.R) x += g.R[off];
+  g.D[off] = x;
+}
+
+// Whether gemm_small_kernel takes the batch: aligned groups of 4 k, and little enough work that the
+// latency of the tiled kernels, which walk all of K in one workgroup, costs more than reading every
+// operand 16 rows at a time. Work in 16 x 16 x 16 blocks: the small kernel takes 2.5 us and 1 us for
+// every 3,200, the tiled ones at least 3.4 us and 0.85 us for every 32 k. (128-wide maps, l <= 3: 32
+// nodes 7.1 -> 3.1 us, 256 nodes 7.3 us either way, 512 nodes 7.6 against 12.7; K = 512 to 896: 32 nodes 27.3
+// -> 7.1 us, 256 nodes 32 against 36.)
+static bool small_ok(const GemmBatch& gb, int n_ranks) {
+  int64_t blocks = 0;
+  int max_k = 0;
+  for (int l = 0; l < n_ranks; ++l) {
+    const GemmRank& g = gb.r[l];
+    if ((g.K & 3) || (g.a_row & 3) || (g.a_comp & 3) || ((uintptr_t)g.A & 15) || ((uintptr_t)g.P & 15) ||
+        (gb.trans_b && ((uintptr_t)g.B & 15)))
+      return false;
+    blocks += (int64_t)((g.M + 15) / 16) * ((g.N + 15) / 16) * ((g.K + 15) / 16);
+    if (g.K > max_k) max_k = g.K;
+  }
+  return blocks <= 3200 + 85 * (int64_t)max_k;
+}
+
+static int launch_small(GemmBatch gb, int n_ranks, hipStream_t s) {
+  int64_t total = 0;
+  int max_k = 0;
+  for (int l = 0; l < n_ranks; ++l) {
+    GemmRank& g = gb.r[l];
+    g.tiles_m = (g.M + 15) / 16;
+    g.tiles_n = (g.N + 15) / 16;
+    g.tile_base = (int32_t)total;
+    total += (int64_t)g.tiles_m * g.tiles_n;
+    if (g.K > max_k) max_k = g.K;
+  }
+  if (total == 0) return FC_OK;
+  gb.n_ranks = n_ranks;
+  gb.total_tiles = (int32_t)total;
+  const dim3 grid((unsigned)total), block(256);
+  // U: the chunks of 16 k that fall to a wave, up to 8
+  const int per = ((max_k + 15) / 16 + 3) / 4;
+  auto launch = [&](auto u) {
+    constexpr int U = decltype(u)::value;
+    if (gb.pair_sum) hipLaunchKernelGGL((gemm_small_kernel<false, true, U>), grid, block, 0, s, gb);
+    else if (gb.trans_b) hipLaunchKernelGGL((gemm_small_kernel<false, false, U>), grid, block, 0, s, gb);
+    else hipLaunchKernelGGL((gemm_small_kernel<true, false, U>), grid, block, 0, s, gb);
+  };
+  if (per <= 1) launch(std::integral_constant<int, 1>{});
+  else if (per <= 2) launch(std::integral_constant<int, 2>{});
+  else if (per <= 4) launch(std::integral_constant<int, 4>{});
+  else launch(std::integral_constant<int, 8>{});
+  FC_LAUNCH_CHECK();
+  return FC_OK;
+}
+
 template <int BM, int BN, int WM, int WN, int NBUF>
 int launch_gemm_cfg(GemmBatch gb, int n_ranks, hipStream_t s) {
   int64_t total = 0;
@@ -732,6 +876,7 @@ int launch_gemm(GemmBatch gb, int n_ranks, hipStream_t s) {
     if (gb.r[l].M < 0) return FC_ERR_SHAPE;
   }
   if (max_m == 0 || max_n == 0 || n_ranks == 0) return FC_OK;
+  if (small_ok(gb, n_ranks)) return launch_small(gb, n_ranks, s);
   if (gb.pair_sum) return launch_pairsum(gb, s);
   if (split_ok(gb, n_ranks)) {
     // 128-column tiles where they fill the chip (two workgroups per CU) and the map is wider than 64;

@@ -596,13 +596,17 @@ def _map_bound(x, w, k):
 
 
 @pytest.mark.parametrize("n,lin,lout,fin,fout,paths", [
-    (1, 0, 0, 32, 4, [1]), (127, 1, 1, 32, 33, [1, 2]), (43, 2, 1, 64, 63, [1, 1, 2]), (129, 0, 0, 96, 65, [1]),
-    (33, 3, 3, 32, 100, [5, 1, 2, 3]), (128, 1, 2, 160, 128, [1, 1]),
+    # little work: 16 x 16 blocks, K below, at and above the 16 k chunks and the waves' shares of them
+    (1, 0, 0, 4, 4, [1]), (17, 2, 2, 12, 20, [1, 2, 1]), (33, 3, 1, 36, 33, [1, 1, 1, 1]),
+    (5, 1, 3, 128, 128, [7, 3]), (64, 0, 0, 512, 16, [1]), (43, 1, 2, 68, 36, [1, 2]),
+    # 64-column tiles
+    (50001, 0, 0, 32, 4, [1]), (6001, 1, 1, 32, 33, [1, 2]), (2203, 2, 1, 64, 63, [1, 1, 2]),
+    (8129, 0, 0, 96, 65, [1]), (2033, 3, 3, 32, 100, [5, 1, 2, 3]), (1128, 1, 2, 160, 128, [1, 1]),
     # enough tiles for 128-column tiles: two column tiles, the second and the last row tile partial
     (40001, 0, 0, 32, 200, [1]), (8201, 3, 3, 32, 132, [1, 2, 1, 1])])
-def test_linear_split_tiles(n, lin, lout, fin, fout, paths):
-    """The split GEMM at the edges of its tiles (rows, columns, K steps), forward with a residual and input
-    gradient, against float64 with an element-wise bound."""
+def test_linear_tiles(n, lin, lout, fin, fout, paths):
+    """The linear maps' kernels at the edges of their tiles (rows, columns, K steps), forward with a residual and
+    input gradient, against float64 with an element-wise bound."""
     ops = _ops()
     g = torch.Generator(device=DEV).manual_seed(n + fout)
     common = min(lin, lout)
@@ -633,9 +637,9 @@ def test_linear_split_tiles(n, lin, lout, fin, fout, paths):
         oo += m * fout if l <= lout else 0
 
 
-@pytest.mark.parametrize("n,fout", [(70, 40), (40000, 136)])
-def test_linear_split_special_values(n, fout):
-    """Infinities and NaN propagate through the split GEMM as IEEE sums (also where a weight is zero), and
+@pytest.mark.parametrize("n,fout", [(70, 40), (20000, 40), (40000, 136)])
+def test_linear_special_values(n, fout):
+    """Infinities and NaN propagate through the linear maps as IEEE sums (also where a weight is zero), and
     operands at both ends of float32's range keep its precision."""
     ops = _ops()
     k = 64
@@ -723,3 +727,20 @@ def test_dense_tiles(n, k, m, act):
     want_gx = 0.125 * (a @ w.double())
     gx_bound = 0.125 * _map_bound(a, w.double().t(), m) + 0.125 * (slack @ w.double().abs())
     assert bool(((gx.double() - want_gx).abs() <= gx_bound)[rows].all())
+
+
+@pytest.mark.parametrize("pairs", [1, 37, 6001])
+def test_dense_bwd_pairs_sizes(pairs):
+    """The pair-summed input gradient with few pairs and with enough for its tiled kernel."""
+    ops = _ops()
+    k = 704
+    g = torch.Generator(device=DEV).manual_seed(pairs)
+    go = torch.randn(2 * pairs, k, device=DEV, generator=g)
+    w = torch.randn(k, 64, device=DEV, generator=g)
+    perm = torch.randperm(2 * pairs, device=DEV, generator=g).to(torch.int32)
+    lo, hi = perm[:pairs].contiguous(), perm[pairs:].contiguous()
+    with torch.no_grad():
+        got = ops.dense_bwd_pairs(go, w, 0.5, lo, hi)
+    a = go[lo.long()].double() + go[hi.long()].double()
+    bound = 0.5 * _map_bound(go[lo.long()].abs().double() + go[hi.long()].abs().double(), w.double().t(), k)
+    assert bool(((got.double() - 0.5 * (a @ w.double())).abs() <= bound).all())
