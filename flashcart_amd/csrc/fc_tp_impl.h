@@ -168,12 +168,13 @@ __device__ __forceinline__ void fill_amat(const float* __restrict__ in2, int64_t
   });
 }
 
-// EG > 1 (convolution with C = 32 or 64 only): EG groups of C lanes share a receiver (block C * EG
+// EG > 1 (convolution with C = 32, 64 or 128 only): EG groups of C lanes share a receiver (block C * EG
 // threads), group g taking the edges e0 + g, e0 + g + EG, ...; the groups' partial sums are added in
 // LDS in group order (so results are reproducible run to run) and stored by group 0. This gives a
-// graph with few receivers and few channels enough waves to hide the gather latency.
-template <int L1, int L2, int LO, bool SYM, bool CONV, bool BC2, int EG = 1>
-__global__ void __launch_bounds__(256) tp_fwd_kernel(TPArgs g) {
+// graph with few receivers and few channels enough waves to hide the gather latency. CW: the widest C
+// of the instantiation (with 128 channels the groups take turns with one LDS buffer of partial sums).
+template <int L1, int L2, int LO, bool SYM, bool CONV, bool BC2, int EG = 1, int CW = 64>
+__global__ void __launch_bounds__(CW * EG > 256 ? CW * EG : 256) tp_fwd_kernel(TPArgs g) {
   // The forward keeps the per-lane coupling matrices: it is bound by the gathered
   // operand stream, and staging the matrices in LDS (as the backward does) measured
   // slower here (chunk barriers and broadcast LDS reads on the critical path).
@@ -181,10 +182,10 @@ __global__ void __launch_bounds__(256) tp_fwd_kernel(TPArgs g) {
   using PL = typename CF::PL;
   constexpr int D1 = CF::D1, D2 = CF::D2, NOUT = CF::NOUT, NP = CF::NP;
   static_assert(EG == 1 || CONV, "edge groups split a receiver's edges");
-  extern __shared__ float part_lds[];  // EG > 1: (EG - 1) x NOUT x C partial sums
+  extern __shared__ float part_lds[];  // EG > 1: (CW > 64 ? 1 : EG - 1) x NOUT x C partial sums
   const int64_t row = CONV ? xcd_row(g.n_rows) : (int64_t)blockIdx.x;
   const int C = g.C;
-  const int grp = EG == 1 ? 0 : (int)threadIdx.x / C;
+  const int grp = EG == 1 ? 0 : CW > 64 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x / C) : (int)threadIdx.x / C;
   const int f = EG == 1 ? (int)threadIdx.x : (int)threadIdx.x % C;
   if (row >= g.n_rows) return;  // uniform over the workgroup
   if (EG == 1 && f >= C) return;
@@ -199,25 +200,28 @@ __global__ void __launch_bounds__(256) tp_fwd_kernel(TPArgs g) {
   if constexpr (CONV) { e0 = g.rowptr[row] + grp; e1 = g.rowptr[row + 1]; }
   EdgeOps<D1, D2, NP> cur, nxt;
   // With edge groups an edge's index differs between groups, so idx_j[e] and its pair slot are
-  // vector loads that the row loads would wait for one edge at a time. Instead the group's lanes
-  // stage the senders and weight rows of its next C edges in LDS (one load each, C edges per wait)
-  // and the loop reads them from there.
-  __shared__ int32_t ix_lds[CONV && EG > 1 ? 2 * EG * 64 : 1];
-  auto stage_idx = [&](int64_t k0) {  // the group's edges k0 .. k0 + C - 1
+  // vector loads that the row loads would wait for one edge at a time. Instead the lanes stage the
+  // senders and weight rows of their group's next SL edges in LDS (one load each, SL edges per wait)
+  // and the loop reads them from there. Staging is private to a wave (a group of two waves stages
+  // them twice), so it needs no barrier in the groups' loops, which differ in length.
+  const int SL = C < 64 ? C : 64;
+  __shared__ int32_t ix_lds[CONV && EG > 1 ? 2 * EG * CW : 1];
+  int32_t* const ix = ix_lds + (CW > 64 ? (int)(threadIdx.x >> 6) : grp) * 128;
+  const int fs = CW > 64 ? f & 63 : f;
+  auto stage_idx = [&](int64_t k0) {  // the group's edges k0 .. k0 + SL - 1
     if constexpr (CONV && EG > 1) {
-      const int64_t e = e0 + (k0 + f) * EG;
+      const int64_t e = e0 + (k0 + fs) * EG;
       if (e < e1) {
-        ix_lds[grp * 128 + f] = g.idx_j[e];
-        ix_lds[grp * 128 + 64 + f] = g.shared_w ? 0 : (int32_t)weight_row(g, e);
+        ix[fs] = g.idx_j[e];
+        ix[64 + fs] = g.shared_w ? 0 : (int32_t)weight_row(g, e);
       }
     }
   };
   auto load_k = [&](int64_t k, EdgeOps<D1, D2, NP>& o) {  // the group's edge k
     const int64_t e = e0 + k * EG;
     if constexpr (CONV && EG > 1) {
-      const int s = (int)(k & (C - 1));  // C is 32 or 64 with edge groups
-      load_edge<D1, D2, NP, CONV, BC2, true, true>(g, e, f1, f2, f, true, o, ix_lds[grp * 128 + s],
-                                                   ix_lds[grp * 128 + 64 + s]);
+      const int s = (int)(k & (SL - 1));  // C is 32, 64 or 128 with edge groups
+      load_edge<D1, D2, NP, CONV, BC2, true, true>(g, e, f1, f2, f, true, o, ix[s], ix[64 + s]);
     } else {
       load_edge<D1, D2, NP, CONV, BC2>(g, e, f1, f2, f, true, o);
     }
@@ -228,7 +232,7 @@ __global__ void __launch_bounds__(256) tp_fwd_kernel(TPArgs g) {
   for (int64_t e = e0; e < e1; e += EG, ++k) {
     cur = nxt;
     if (e + EG < e1) {
-      if (((k + 1) & (C - 1)) == 0) stage_idx(k + 1);
+      if (((k + 1) & (SL - 1)) == 0) stage_idx(k + 1);
       load_k(k + 1, nxt);
     }
     static_for<NP>([&](auto ic) {
@@ -242,7 +246,22 @@ __global__ void __launch_bounds__(256) tp_fwd_kernel(TPArgs g) {
       for (int a = 0; a < T::NO; ++a) acc[PL::out_index(i, a)] = fmaf(cur.w[i], t[a], acc[PL::out_index(i, a)]);
     });
   }
-  if constexpr (EG > 1) {
+  if constexpr (EG > 1 && CW > 64) {
+#pragma unroll 1
+    for (int q = 1; q < EG; ++q) {
+      if (grp == q) {
+#pragma unroll
+        for (int k = 0; k < NOUT; ++k) part_lds[k * C + f] = acc[k];
+      }
+      __syncthreads();
+      if (grp == 0) {
+#pragma unroll
+        for (int k = 0; k < NOUT; ++k) acc[k] += part_lds[k * C + f];
+      }
+      __syncthreads();
+    }
+    if (grp > 0) return;
+  } else if constexpr (EG > 1) {
     if (grp > 0) {
 #pragma unroll
       for (int k = 0; k < NOUT; ++k) part_lds[((grp - 1) * NOUT + k) * C + f] = acc[k];
@@ -517,7 +536,7 @@ __global__ void __launch_bounds__(C * EG, 2) tp_bwd_conv_kernel(TPArgs g) {
   constexpr int NWG = C >= 64 ? C / 64 : 1;          // waves per group
   constexpr int R2 = pow2_at_least(D2), SH2 = log2_exact(GW) - log2_exact(R2);
   constexpr int CH = bwd_conv_chunk<L1, L2, LO, SYM>();
-  static_assert((C == 32 || C % 64 == 0) && C <= 256 && T % 64 == 0 && T <= 256, "whole waves of whole groups");
+  static_assert((C == 32 || C % 64 == 0) && C <= 256 && T % 64 == 0 && T <= 512, "whole waves of whole groups");
   static_assert(CH % (2 * EG) == 0, "every full chunk gives each group an even number of edges");
   static_assert(2 * CH * AL::total * 4 <= 65536, "coupling-matrix chunks exceed the LDS budget");
   constexpr int64_t SW = (int64_t)NP * C, S1 = (int64_t)D1 * C;
@@ -528,7 +547,8 @@ __global__ void __launch_bounds__(C * EG, 2) tp_bwd_conv_kernel(TPArgs g) {
   const int64_t row = xcd_row(g.n_rows);
   if (row >= g.n_rows) return;
   const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
-  const int grp = EG == 1 ? 0 : t / C, f = EG == 1 ? t : t % C;
+  // (a group of whole waves is the same for all lanes: in a scalar register its edges' addresses are too)
+  const int grp = EG == 1 ? 0 : C >= 64 ? __builtin_amdgcn_readfirstlane(t / C) : t / C, f = EG == 1 ? t : t % C;
   const int wig = C >= 64 ? f >> 6 : 0;  // wave within the group
   const int64_t e0 = g.rowptr[row], e1 = g.rowptr[row + 1];
   if (e0 >= e1) return;  // uniform over the workgroup: no barrier is skipped by a part of it
@@ -747,7 +767,8 @@ __global__ void __launch_bounds__(C * EG, 2) tp_bwd_send_kernel(TPArgs g) {
   const int64_t row = xcd_row(g.n_rows);  // the sender
   if (row >= g.n_rows) return;
   const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
-  const int grp = EG == 1 ? 0 : t / C, f = EG == 1 ? t : t % C;
+  // (a group of whole waves is the same for all lanes: in a scalar register its edges' addresses are too)
+  const int grp = EG == 1 ? 0 : C >= 64 ? __builtin_amdgcn_readfirstlane(t / C) : t / C, f = EG == 1 ? t : t % C;
   const int wig = C >= 64 ? f >> 6 : 0;
   const int64_t k0 = g.sptr[row], k1 = g.sptr[row + 1];
   const float alpha = scale_of(g);
@@ -977,12 +998,23 @@ __global__ void __launch_bounds__(256) tp_bwd_rows_kernel(TPArgs g) {
   }
 }
 
-// Edge groups per receiver of the convolution kernels with C <= 64 channels: enough waves to
+// Whether the 128-channel convolution kernels of a product come with four edge groups (512 threads, at
+// most 256 registers a lane): those whose output rows leave room for the operands of two edges.
+template <int L1, int L2, int LO, bool SYM>
+constexpr bool wide_groups() {
+  return !SYM && L1 <= 3 && L2 >= 1 && L2 <= 3 && LO <= 3 && TPConfig<L1, L2, LO, SYM>::NOUT <= 80;
+}
+
+// Edge groups per receiver of the convolution kernels with C <= 128 channels: enough waves to
 // occupy the GPU (about four per SIMD, 4,096) when the graph has few receivers, at most 256
-// threads per workgroup and at most half the mean in-degree per group.
+// threads per workgroup (512 with 128 channels) and at most half the mean in-degree per group.
 inline int conv_edge_groups(int64_t n_rows, int64_t n_edges, int C) {
   // 512 receivers x 8 edges with 32 channels: 29.0 us per forward + backward with four groups,
   // 32.4 us with eight (measured on the standalone product of the benchmark's first configuration)
+  // 128 channels, 42 edges a receiver, 2x3->3 product, forward / backward op: 32 receivers 69 / 156 us with one
+  // group, 39 / 66 us with four; 256: 77 / 181 and 37 / 87; 512: 87 / 197 and 60 / 165; 768: 95 / 238 and
+  // 88 / 240; 1,024: 109 / 299 and 120 / 319
+  if (C == 128) return n_rows < 768 && 8 * n_rows <= n_edges ? 4 : 1;
   const int max_eg = C == 32 || C == 64 ? 4 : 1;
   int eg = C == 32 ? 2 : 1;
   const double deg = n_rows > 0 ? (double)n_edges / (double)n_rows : 0.0;
@@ -1021,6 +1053,12 @@ constexpr int kSendNotApplicable = -100;
 template <int L1, int L2, int LO, bool SYM, int EG>
 void launch_fwd_groups(const TPArgs& g, dim3 grid, hipStream_t stream) {
   using CF = TPConfig<L1, L2, LO, SYM>;
+  if (g.C == 128) {
+    if constexpr (EG == 4 && wide_groups<L1, L2, LO, SYM>())
+      hipLaunchKernelGGL((tp_fwd_kernel<L1, L2, LO, SYM, true, true, EG, 128>), grid, dim3(g.C * EG),
+                         sizeof(float) * (size_t)CF::NOUT * g.C, stream, g);
+    return;
+  }
   const size_t lds = sizeof(float) * (size_t)(EG - 1) * CF::NOUT * g.C;
   hipLaunchKernelGGL((tp_fwd_kernel<L1, L2, LO, SYM, true, true, EG>), grid, dim3(g.C * EG), lds, stream, g);
 }
@@ -1034,7 +1072,9 @@ int launch_tp(const TPArgs& g, bool conv, bool bwd, hipStream_t stream) {
   dim3 grid((unsigned)(conv ? xcd_grid(g.n_rows) : g.n_rows)), block(threads);
   const bool bc2 = conv && g.F2 == 1;
   // edge groups for few-channel convolutions (one in2 channel, full-width in1)
-  const int eg0 = (bc2 && g.F1 == g.C && (g.C == 32 || g.C == 64)) ? conv_edge_groups(g.n_rows, g.n_edges, g.C) : 1;
+  const int eg0 = (bc2 && g.F1 == g.C && (g.C == 32 || g.C == 64 || (g.C == 128 && wide_groups<L1, L2, LO, SYM>())))
+                      ? conv_edge_groups(g.n_rows, g.n_edges, g.C)
+                      : 1;
   if (bwd) {
     const bool reduce = (g.grad_in1 && g.F1 == 1 && g.C > 1) || (g.grad_in2 && g.F2 == 1 && g.C > 1);
     const size_t per_edge = reduce ? sizeof(float) * (threads / 64) * (ncomp(L1) + ncomp(L2)) : 0;
@@ -1063,7 +1103,9 @@ int launch_tp(const TPArgs& g, bool conv, bool bwd, hipStream_t stream) {
           (g.C == 32 || g.C == 64 || g.C == 128)) {  // per-edge weights: the kernel reads w[e] rows
         bool done = false;
         if (g.C == 128) {
-          done = launch_bwd_conv<L1, L2, LO, SYM, 128, 1>(g, grid, stream);
+          if constexpr (wide_groups<L1, L2, LO, SYM>())
+            done = eg0 >= 4 && launch_bwd_conv<L1, L2, LO, SYM, 128, 4>(g, grid, stream);
+          done = done || launch_bwd_conv<L1, L2, LO, SYM, 128, 1>(g, grid, stream);
         } else if (g.C == 64) {
           done = (eg0 >= 4 && launch_bwd_conv<L1, L2, LO, SYM, 64, 4>(g, grid, stream)) ||
                  (eg0 >= 2 && launch_bwd_conv<L1, L2, LO, SYM, 64, 2>(g, grid, stream)) ||

@@ -744,3 +744,31 @@ def test_dense_bwd_pairs_sizes(pairs):
     a = go[lo.long()].double() + go[hi.long()].double()
     bound = 0.5 * _map_bound(go[lo.long()].abs().double() + go[hi.long()].abs().double(), w.double().t(), k)
     assert bool(((got.double() - 0.5 * (a @ w.double())).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("l1,l2,lo", [(2, 3, 3), (0, 3, 3)])
+@pytest.mark.parametrize("degrees", [(9, 0, 41, 8), (300, 65, 1), (8,) * 40, (7,) * 40, (17, 16, 15) * 255])
+def test_tp_conv_edge_groups_128(l1, l2, lo, degrees):
+    """128-channel convolutions whose receivers are shared by four edge groups (two waves each): groups of
+    unequal length, empty receivers, more edges than a wave stages indices of (64 a group), mean degrees around the 8
+    where the groups begin and up to the 768 receivers where they end; all gradients, against float64."""
+    C = 128
+    n = len(degrees)
+    ei = random_csr_graph(n, degrees, seed=n, allow_self=True)
+    g = torch.Generator().manual_seed(n + l1)
+    e = ei.shape[1]
+    from oracle.cartesian import enumerate_paths
+    P = len(enumerate_paths(l1, l2, lo, False))
+    leaves64 = [torch.randn(*s, generator=g, dtype=torch.float64).requires_grad_(True)
+                for s in ((n, (l1 + 1) ** 2 * C), (e, (l2 + 1) ** 2), (e, P * C))]
+    ref = O.tensor_product(*leaves64, ei[0], ei[1], l1, l2, lo, C, 1)
+    go = torch.randn(ref.shape, generator=g, dtype=torch.float64)
+    want = torch.autograd.grad(ref, leaves64, go)
+    from flashcart_amd import o3
+    tp = o3.TensorProduct(l1, l2, lo, C, 1)
+    leaves = [t.detach().float().to(DEV).requires_grad_(True) for t in leaves64]
+    out = tp(*leaves, ei[0].to(DEV), ei[1].to(DEV))
+    got = torch.autograd.grad(out, leaves, go.float().to(DEV))
+    assert_close(out, ref, 2e-5, 2e-5 * (float(ref.abs().max()) + 1), "forward")
+    for k, (a, b) in enumerate(zip(got, want)):
+        assert_close(a, b, 2e-5, 2e-5 * (float(b.abs().max()) + 1), f"gradient {k}")
