@@ -772,3 +772,56 @@ def test_tp_conv_edge_groups_128(l1, l2, lo, degrees):
     assert_close(out, ref, 2e-5, 2e-5 * (float(ref.abs().max()) + 1), "forward")
     for k, (a, b) in enumerate(zip(got, want)):
         assert_close(a, b, 2e-5, 2e-5 * (float(b.abs().max()) + 1), f"gradient {k}")
+
+
+@pytest.mark.parametrize("n", [1, 7, 33, 257, 5003])
+@pytest.mark.parametrize("k,m,act", [(3, 4, 0), (130, 65, 1), (64, 128, 0), (200, 64, 1)])
+def test_wgrad_tiles(n, k, m, act):
+    """Dense weight and bias gradients at row counts around the kernel's groups of 8, steps of 32 and parts of
+    256, and column counts around its tiles, with an element-wise bound; then with an infinity and a NaN in
+    the rows, which reach the sums they reach in IEEE arithmetic."""
+    ops = _ops()
+    g = torch.Generator(device=DEV).manual_seed(n + m)
+    go, pre, x = (torch.randn(n, c, device=DEV, generator=g) for c in (m, m, k))
+    a = go.double()
+    if act:
+        z = pre.double().requires_grad_(True)
+        (dz,) = torch.autograd.grad(O.silu(z).sum(), z)
+        a = a * dz
+    slack = 2.0 ** -20 * a.abs() if act else 0.0 * a  # the derivative's exp
+    with torch.no_grad():
+        gw, gb = ops.dense_wgrad(go, pre if act else None, act, x, 0.5, True, True)
+    bound = 0.5 * _map_bound(a.t(), x.double().t(), n) + 0.5 * (slack.t() @ x.double().abs())
+    assert bool(((gw.double() - 0.5 * (a.t() @ x.double())).abs() <= bound).all())
+    assert bool(((gb.double() - a.sum(0)).abs() <= (n / 8 + 8) * 2.0 ** -23 * a.abs().sum(0) + slack.sum(0)).all())
+    go[n // 2, 0] = float("inf")
+    x[n - 1, k - 1] = float("nan")
+    with torch.no_grad():
+        gw, _ = ops.dense_wgrad(go, pre if act else None, act, x, 0.5, True, False)
+    a = go.double() * dz if act else go.double()
+    want = 0.5 * (a.t() @ x.double())
+    assert torch.equal(gw.isnan(), want.isnan()) and torch.equal(gw.isinf(), want.isinf())
+    ok = want.isfinite()
+    assert bool(((gw.double() - want).abs() <= bound)[ok].all())
+
+
+@pytest.mark.parametrize("n,lin,lout,fin,fout,paths", [(1, 3, 3, 4, 4, [1] * 4), (37, 3, 2, 33, 65, [1, 2, 1, 1]),
+                                                       (1001, 3, 3, 64, 128, [2, 1, 1, 1])])
+def test_linear_wgrad_tiles(n, lin, lout, fin, fout, paths):
+    """Rows in place in the packed features (components 1, 3, 5, 7 to a node) across the kernel's steps."""
+    ops = _ops()
+    g = torch.Generator(device=DEV).manual_seed(n)
+    x = torch.randn(n, sum((2 * l + 1) * fin * paths[l] for l in range(lin + 1)), device=DEV, generator=g)
+    go = torch.randn(n, (lout + 1) ** 2 * fout, device=DEV, generator=g)
+    common = min(lin, lout)
+    ws = [torch.empty(fout, fin * paths[l], device=DEV) for l in range(common + 1)]
+    with torch.no_grad():
+        got = ops.linear_wgrad(go, x, ws, lin, lout, fin, fout, paths, [1.0] * (common + 1), 1.0, [True] * (common + 1))
+    io = oo = 0
+    for l in range(common + 1):
+        m, k = 2 * l + 1, fin * paths[l]
+        a = go[:, oo:oo + m * fout].reshape(n * m, fout).double()
+        b = x[:, io:io + m * k].reshape(n * m, k).double()
+        assert bool(((got[l].double() - a.t() @ b).abs() <= _map_bound(a.t(), b.t(), n * m)).all()), f"rank {l}"
+        io += m * k
+        oo += m * fout
