@@ -15,6 +15,8 @@ raises otherwise; there is no CPU path.
 from __future__ import annotations
 
 import contextlib
+import functools
+import inspect
 from typing import List, Optional, Tuple
 
 import torch
@@ -108,6 +110,7 @@ def _i32(name: str, t: Optional[Tensor]) -> Optional[Tensor]:
     return t.contiguous()
 
 
+@functools.lru_cache(maxsize=256)
 def _tp_out_dim(in1_l_max, in2_l_max, out_l_max, in1_features, in2_features, symmetric, reduced) -> int:
     counts, _ = count_output_paths(in1_l_max, in2_l_max, out_l_max, symmetric)
     c = max(in1_features, in2_features)
@@ -153,6 +156,101 @@ def param_alias(t: Optional[Tensor]) -> Optional[Tensor]:
     return t
 
 
+def _c(name: str):
+    """A query of torch's C extension by its dotted name, or None in a build without it."""
+    obj = torch._C
+    for part in name.split("."):
+        obj = getattr(obj, part, None)
+    return obj
+
+
+# What else may be looking at a call: dispatch and function modes (fake tensors, tracers), functorch
+# transforms (vmap, grad), a jit trace, the profiler. A build that cannot say is assumed to look.
+_QUERIES = tuple(_c(n) for n in ("_len_torch_dispatch_stack", "_len_torch_function_stack",
+                                 "_functorch.peek_interpreter_stack", "_get_tracing_state",
+                                 "_autograd._profiler_enabled"))
+_PLAIN = (Tensor, torch.nn.Parameter)
+# The exact types an argument may have to skip the registry's conversions, by annotation.
+_EXACT = {"Tensor": _PLAIN, "Optional[Tensor]": _PLAIN + (type(None),), "int": (int,), "bool": (bool,),
+          "float": (float,), "List[int]": (list, tuple), "List[float]": (list, tuple)}
+_EXACT_ITEM = {"List[int]": int, "List[float]": float}
+
+
+def _observed() -> bool:
+    if torch.compiler.is_compiling() or None in _QUERIES:
+        return True
+    modes, functions, functorch, tracing, profiler = _QUERIES
+    return bool(modes() or functions() or functorch() is not None or tracing() is not None or profiler()
+                or getattr(torch.autograd.forward_ad, "_current_level", 0) >= 0)
+
+
+class Operator:
+    """A registered operator (``torch.ops.flashcart.*``) and its Python callable. Calling it runs the
+    implementation, under an ``autograd.Function`` of the same formula where a gradient is wanted, without
+    the operator registry's argument handling, which costs more host time (100 us for the 24 arguments of
+    ``tp_fwd``) than the kernels of a small call take. Anything that has to see or rewrite the operator itself
+    (``_observed``, tensor subclasses, tensors that are not on a GPU) and every call that the registry would
+    convert or refuse (keywords, arguments of other types or counts) goes through the registered operator;
+    both run the same implementation and the same backward."""
+
+    def __init__(self, name: str, impl):
+        self.op = torch.library.custom_op(name, mutates_args=())(impl)
+        self.impl = impl
+        self.function = None
+        params = tuple(inspect.signature(impl).parameters.values())
+        self.defaults = tuple(q.default for q in params)
+        self.required = sum(q.default is inspect.Parameter.empty for q in params)
+        self.exact = tuple(_EXACT[q.annotation] for q in params)
+        self.items = tuple((k, _EXACT_ITEM[q.annotation]) for k, q in enumerate(params)
+                           if q.annotation in _EXACT_ITEM)
+        functools.update_wrapper(self, impl)
+
+    def register_fake(self, fn):
+        return self.op.register_fake(fn)
+
+    def register_autograd(self, backward, setup_context):
+        self.op.register_autograd(backward, setup_context=setup_context)
+        impl = self.impl
+
+        class Direct(torch.autograd.Function):
+            @staticmethod
+            def forward(ctx, *inputs):
+                output = impl(*inputs)
+                setup_context(ctx, inputs, output)
+                return output
+
+            @staticmethod
+            def backward(ctx, *grads):
+                return backward(ctx, *grads)
+
+        Direct.__name__ = self.__name__
+        self.function = Direct
+
+    def _direct(self, args) -> bool:
+        """Whether ``args`` (positional) need nothing that the registered operator would do."""
+        if not self.required <= len(args) <= len(self.exact):
+            return False
+        for a, exact in zip(args, self.exact):
+            if type(a) not in exact or (exact[0] is Tensor and a is not None and not a.is_cuda):
+                return False
+        return all(type(x) is item for k, item in self.items if k < len(args) for x in args[k])
+
+    def __call__(self, *args, **kwargs):
+        if kwargs or _observed() or not self._direct(args):
+            return self.op(*args, **kwargs)
+        args += self.defaults[len(args):]
+        if torch.is_grad_enabled() and any(isinstance(a, Tensor) and a.requires_grad for a in args):
+            if self.function is None:
+                return self.op(*args)
+            return self.function.apply(*args)
+        return self.impl(*args)
+
+
+def operator(name: str):
+    """Register the decorated implementation as ``torch.ops.flashcart.<name>``."""
+    return lambda impl: Operator(name, impl)
+
+
 def _register_autograd(op, backward, setup_context) -> None:
     """``op.register_autograd`` with ``ctx.needs_input_grad`` narrowed, while the backward
     runs, to the inputs the running backward pass will actually use.
@@ -194,9 +292,17 @@ def _register_autograd(op, backward, setup_context) -> None:
     op.register_autograd(bwd, setup_context=setup)
 
 
+@functools.lru_cache(maxsize=256)
+def _n_paths(in1_l_max: int, in2_l_max: int, out_l_max: int, symmetric: bool) -> int:
+    return count_output_paths(in1_l_max, in2_l_max, out_l_max, symmetric)[1]
+
+
+_standard_meta = functools.lru_cache(maxsize=256)(lambda *cfg: tp_meta(*cfg))  # (read only: shared by calls)
+
+
 def _check_tp_meta(cfg, in1_offs, in2_offs, out_sizes, n_paths_per_l, n_total_paths) -> None:
     """The kernels implement the standard contiguous layout only; reject any other."""
-    want = tp_meta(*cfg)
+    want = _standard_meta(*cfg)
     got = (list(in1_offs), list(in2_offs), list(out_sizes), list(n_paths_per_l), int(n_total_paths))
     names = ("in1_offs", "in2_offs", "out_sizes", "n_paths_per_l", "n_total_paths")
     for name, g, w in zip(names, got, want):
@@ -212,7 +318,7 @@ def _check_tp_meta(cfg, in1_offs, in2_offs, out_sizes, n_paths_per_l, n_total_pa
 # Eq. (1) expansion
 # ---------------------------------------------------------------------------
 
-@torch.library.custom_op("flashcart::irreps_fwd", mutates_args=())
+@operator("flashcart::irreps_fwd")
 def irreps_fwd(x: Tensor, l_max: int) -> Tensor:
     x = _lib.contig("x", x)
     out = x.new_empty(x.shape[0], (l_max + 1) ** 2)
@@ -225,7 +331,7 @@ def _(x, l_max):
     return x.new_empty(x.shape[0], (l_max + 1) ** 2)
 
 
-@torch.library.custom_op("flashcart::irreps_bwd", mutates_args=())
+@operator("flashcart::irreps_bwd")
 def irreps_bwd(grad_output: Tensor, x: Tensor, l_max: int) -> Tensor:
     g = _lib.contig("grad_output", grad_output)
     x = _lib.contig("x", x)
@@ -239,7 +345,7 @@ def _(grad_output, x, l_max):
     return torch.empty_like(x)
 
 
-@torch.library.custom_op("flashcart::irreps_dbwd", mutates_args=())
+@operator("flashcart::irreps_dbwd")
 def irreps_dbwd(grad_output: Tensor, x: Tensor, v: Tensor, l_max: int) -> Tuple[Tensor, Tensor]:
     """Backward of irreps_bwd along v (reference flashcart::irreps_dbwd, o3/_irreps.py:146-176):
     (d grad_output = J(x) v, d x = sum_a grad_output_a H_a(x) v)."""
@@ -278,7 +384,7 @@ _register_autograd(irreps_fwd, _irreps_backward, _irreps_setup)
 # Radial basis and cutoff envelope
 # ---------------------------------------------------------------------------
 
-@torch.library.custom_op("flashcart::radial_fwd", mutates_args=())
+@operator("flashcart::radial_fwd")
 def radial_fwd(d: Tensor, basis: int, n_radial: int, r_min: float, r_max: float, poly_order: int) -> Tuple[Tensor, Tensor]:
     """(feats (n, n_radial) or empty when basis is NONE, env (n,) or empty when poly_order == 0)."""
     d = _lib.contig("distances", d)
@@ -298,7 +404,7 @@ def _(d, basis, n_radial, r_min, r_max, poly_order):
             d.new_empty(n) if poly_order > 0 else d.new_empty(0))
 
 
-@torch.library.custom_op("flashcart::radial_bwd", mutates_args=())
+@operator("flashcart::radial_bwd")
 def radial_bwd(d: Tensor, g_feats: Optional[Tensor], g_env: Optional[Tensor], basis: int, n_radial: int,
                r_min: float, r_max: float, poly_order: int) -> Tensor:
     d = _lib.contig("distances", d)
@@ -368,7 +474,7 @@ def shift_vectors(cell: Tensor, shifts: Tensor, idx_i: Optional[Tensor], batch: 
     return out
 
 
-@torch.library.custom_op("flashcart::edge_geometry", mutates_args=())
+@operator("flashcart::edge_geometry")
 def edge_geometry(positions: Optional[Tensor], shift_vec: Optional[Tensor], idx_i: Tensor, idx_j: Tensor,
                   vectors: Optional[Tensor], rowptr: Optional[Tensor], sender_perm: Optional[Tensor],
                   sender_ptr: Optional[Tensor], l_max: int, basis: int, n_radial: int, r_min: float, r_max: float,
@@ -403,7 +509,7 @@ def _(positions, shift_vec, idx_i, idx_j, vectors, rowptr, sender_perm, sender_p
             ref.new_empty(E) if poly_order > 0 else ref.new_empty(0))
 
 
-@torch.library.custom_op("flashcart::edge_geometry_bwd", mutates_args=())
+@operator("flashcart::edge_geometry_bwd")
 def edge_geometry_bwd(g_attrs: Optional[Tensor], g_feats: Optional[Tensor], g_env: Optional[Tensor],
                       positions: Optional[Tensor], shift_vec: Optional[Tensor], idx_i: Tensor, idx_j: Tensor,
                       vectors: Optional[Tensor], rowptr: Optional[Tensor], sender_perm: Optional[Tensor],
@@ -521,7 +627,7 @@ def _check_tp_inputs(in1, in2, weights, idx_i, idx_j, in1_l_max, in2_l_max, out_
                      in2_features, symmetric_product, shared_weights, paired=False):
     conv = idx_i is not None and idx_j is not None
     c = max(in1_features, in2_features)
-    _, n_paths = count_output_paths(in1_l_max, in2_l_max, out_l_max, symmetric_product)
+    n_paths = _n_paths(in1_l_max, in2_l_max, out_l_max, bool(symmetric_product))
     if in1.shape[-1] != (in1_l_max + 1) ** 2 * in1_features or in2.shape[-1] != (in2_l_max + 1) ** 2 * in2_features:
         raise ValueError("tensor-product input widths do not match the configuration.")
     items = idx_i.shape[0] if conv else in1.shape[0]
@@ -542,7 +648,7 @@ def _check_tp_inputs(in1, in2, weights, idx_i, idx_j, in1_l_max, in2_l_max, out_
     return conv
 
 
-@torch.library.custom_op("flashcart::tp_fwd", mutates_args=())
+@operator("flashcart::tp_fwd")
 def tp_fwd(in1: Tensor, in2: Tensor, weights: Tensor, idx_i: Optional[Tensor], idx_j: Optional[Tensor],
            in1_l_max: int, in2_l_max: int, out_l_max: int, in1_features: int, in2_features: int,
            symmetric_product: bool, shared_weights: bool, in1_offs: List[int], in2_offs: List[int],
@@ -582,11 +688,11 @@ def _(in1, in2, weights, idx_i, idx_j, in1_l_max, in2_l_max, out_l_max, in1_feat
       symmetric_product, shared_weights, in1_offs, in2_offs, out_sizes, n_paths_per_l, n_total_paths,
       reduce_paths=False, rowptr=None, sender_perm=None, sender_ptr=None, alpha=1.0, pair_slot=None,
       alpha_div=None):
-    return in1.new_empty(in1.shape[0], _tp_out_dim(in1_l_max, in2_l_max, out_l_max, in1_features, in2_features,
-                                                   symmetric_product, reduce_paths))
+    return in1.new_empty(in1.shape[0], _tp_out_dim.__wrapped__(  # (not cached: a tracer's symbols may come here)
+        in1_l_max, in2_l_max, out_l_max, in1_features, in2_features, symmetric_product, reduce_paths))
 
 
-@torch.library.custom_op("flashcart::tp_bwd", mutates_args=())
+@operator("flashcart::tp_bwd")
 def tp_bwd(grad_out: Tensor, in1: Tensor, in2: Tensor, weights: Tensor, idx_i: Optional[Tensor],
            idx_j: Optional[Tensor], in1_l_max: int, in2_l_max: int, out_l_max: int, in1_features: int,
            in2_features: int, symmetric_product: bool, shared_weights: bool, in1_offs: List[int],
@@ -737,7 +843,7 @@ def _pad_ranks(weights):
     return ws
 
 
-@torch.library.custom_op("flashcart::equiv_linear_fwd", mutates_args=())
+@operator("flashcart::equiv_linear_fwd")
 def linear_fwd_op(x: Tensor, w0: Tensor, w1: Optional[Tensor], w2: Optional[Tensor], w3: Optional[Tensor],
                   w4: Optional[Tensor], in_l_max: int, out_l_max: int, in_features: int, out_features: int, in_paths: List[int],
                   scale: List[float], alpha: float = 1.0, residual: Optional[Tensor] = None) -> Tensor:
@@ -764,7 +870,7 @@ def _(x, w0, w1, w2, w3, w4, in_l_max, out_l_max, in_features, out_features, in_
     return x.new_empty(x.shape[0], out_dim)
 
 
-@torch.library.custom_op("flashcart::equiv_linear_dgrad", mutates_args=())
+@operator("flashcart::equiv_linear_dgrad")
 def linear_bwd_op(grad_out: Tensor, w0: Tensor, w1: Optional[Tensor], w2: Optional[Tensor], w3: Optional[Tensor],
                   w4: Optional[Tensor], in_l_max: int, out_l_max: int, in_features: int, out_features: int, in_paths: List[int],
                   scale: List[float], alpha: float = 1.0, residual: Optional[Tensor] = None) -> Tensor:
@@ -1180,7 +1286,7 @@ linear_bwd_ref.register_autograd(_linear_bwd_ref_backward, setup_context=_linear
 # Dense layer with optional rescaled-SiLU epilogue (radial / readout MLPs)
 # ---------------------------------------------------------------------------
 
-@torch.library.custom_op("flashcart::dense_fwd", mutates_args=())
+@operator("flashcart::dense_fwd")
 def dense_fwd(x: Tensor, weight: Tensor, bias: Optional[Tensor], scale: float, act: int) -> Tuple[Tensor, Tensor]:
     """(activated output, pre-activation (empty when act == 0))."""
     x = _lib.contig("x", x)
@@ -1204,7 +1310,7 @@ def _(x, weight, bias, scale, act):
     return x.new_empty(*x.shape[:-1], m), (x.new_empty(*x.shape[:-1], m) if act else x.new_empty(0))
 
 
-@torch.library.custom_op("flashcart::dense_bwd", mutates_args=())
+@operator("flashcart::dense_bwd")
 def dense_bwd(grad_out: Tensor, pre: Tensor, weight: Tensor, scale: float, act: int) -> Tensor:
     go = _lib.contig("grad_out", grad_out)
     w = _lib.contig("weight", weight)
@@ -1351,7 +1457,7 @@ def _radial_mlp_check(x: Tensor, w0: Tensor, w1: Tensor) -> int:
     return n_in
 
 
-@torch.library.custom_op("flashcart::radial_mlp_fwd", mutates_args=())
+@operator("flashcart::radial_mlp_fwd")
 def radial_mlp_fwd(x: Tensor, w0: Tensor, s0: float, w1: Tensor, s1: float, w2: Tensor, s2: float) -> Tensor:
     """s2 silu(s1 silu(s0 x W0^T) W1^T) W2^T in one pass (``fc_radial_mlp_fwd``); the hidden
     activations are not returned (the backward recomputes them)."""
@@ -1389,7 +1495,7 @@ def radial_mlp_bwd_pairsum(grad_h2: Tensor, x: Tensor, w0: Tensor, s0: float, w1
     return gx.reshape(x.shape)
 
 
-@torch.library.custom_op("flashcart::radial_mlp_bwd", mutates_args=())
+@operator("flashcart::radial_mlp_bwd")
 def radial_mlp_bwd(grad_h2: Tensor, x: Tensor, w0: Tensor, s0: float, w1: Tensor, s1: float) -> Tensor:
     """dL/dx of the radial MLP's hidden part from dL/dh2 (``fc_radial_mlp_bwd``)."""
     x = _lib.contig("x", x)
@@ -1519,7 +1625,7 @@ def dense_wgrad(grad_out: Tensor, pre: Optional[Tensor], act: int, x: Tensor, sc
 # Segment sum over contiguous sorted segments (per-graph energies)
 # ---------------------------------------------------------------------------
 
-@torch.library.custom_op("flashcart::segment_sum", mutates_args=())
+@operator("flashcart::segment_sum")
 def segment_sum(src: Tensor, ptr: Tensor, index: Tensor) -> Tensor:
     """dst[s] = sum(src[ptr[s]:ptr[s+1]]); ``index`` (row -> segment) is used by the backward."""
     s = _lib.contig("src", src)
@@ -1553,7 +1659,7 @@ _register_autograd(segment_sum, _seg_backward, _seg_setup)
 # Invariant RMS normalisation
 # ---------------------------------------------------------------------------
 
-@torch.library.custom_op("flashcart::rms_norm", mutates_args=())
+@operator("flashcart::rms_norm")
 def rms_norm(x: Tensor, weight: Tensor, l_max: int, eps: float) -> Tuple[Tensor, Tensor]:
     """(out, scale): out_l = x_l * (m + eps)^-1/2 * weight[l] with m the per-node mean of the
     rank-weighted invariants (reference src/flashcart/nn/layers.py:494-528, no centering)."""
@@ -1575,7 +1681,7 @@ def _(x, weight, l_max, eps):
     return torch.empty_like(x), x.new_empty(x.shape[0])
 
 
-@torch.library.custom_op("flashcart::rms_norm_bwd", mutates_args=())
+@operator("flashcart::rms_norm_bwd")
 def rms_norm_bwd(grad_out: Tensor, x: Tensor, weight: Tensor, scale: Tensor, l_max: int) -> Tensor:
     go = _lib.contig("grad_out", grad_out)
     x = _lib.contig("x", x)
@@ -1632,7 +1738,7 @@ _register_autograd(rms_norm, _rms_backward, _rms_setup)
 # Rank-wise gating
 # ---------------------------------------------------------------------------
 
-@torch.library.custom_op("flashcart::gate", mutates_args=())
+@operator("flashcart::gate")
 def gate(values: Tensor, pre: Tensor, l_max: int, act: int) -> Tensor:
     """values[n, (l, a), c] * act(pre[n, l, c]); act 0 identity, 1 rescaled sigmoid
     (reference src/flashcart/nn/layers.py:609-635)."""
@@ -1652,7 +1758,7 @@ def _(values, pre, l_max, act):
     return torch.empty_like(values)
 
 
-@torch.library.custom_op("flashcart::gate_bwd", mutates_args=())
+@operator("flashcart::gate_bwd")
 def gate_bwd(grad_out: Tensor, values: Tensor, pre: Tensor, l_max: int, act: int, need_values: bool,
              need_pre: bool) -> Tuple[Tensor, Tensor]:
     go = _lib.contig("grad_out", grad_out)

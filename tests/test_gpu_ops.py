@@ -825,3 +825,71 @@ def test_linear_wgrad_tiles(n, lin, lout, fin, fout, paths):
         assert bool(((got[l].double() - a.t() @ b).abs() <= _map_bound(a.t(), b.t(), n * m)).all()), f"rank {l}"
         io += m * k
         oo += m * fout
+
+
+def _route_call(kind):
+    """(operator, arguments) of one call with gradients through every differentiable input."""
+    ops = _ops()
+    gen = torch.Generator().manual_seed(11)
+
+    def t(*shape):
+        return torch.randn(*shape, generator=gen).to(DEV).requires_grad_(True)
+
+    if kind == "conv":
+        i, j = random_csr_graph(9, [4, 0, 3], seed=3)
+        i, j = i.to(DEV).int(), j.to(DEV).int()
+        n_paths = ops._n_paths(1, 1, 1, False)
+        meta = ops.tp_meta(1, 1, 1, 8, 1, False, False)
+        return ops.tp_fwd, (t(9, 32), t(i.numel(), 4), t(i.numel(), 8 * n_paths), i, j, 1, 1, 1, 8, 1, False, False, *meta)
+    if kind == "dense":
+        return ops.dense_fwd, (t(13, 8), t(16, 8), None, 0.3, 1)
+    if kind == "norm":
+        return ops.rms_norm, (t(7, 9 * 8), t(3, 8), 2, 1e-5)
+    return ops.irreps_fwd, (unit_vectors(17, seed=2).float().to(DEV).requires_grad_(True), 2)
+
+
+def _route_results(fn, args):
+    """Outputs, gradients and second derivatives of a call, and the tensors it saves."""
+    saved = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda s: saved.append(tuple(s.shape)) or s, lambda s: s):
+        out = fn(*args)
+    outs = [o for o in (out if isinstance(out, tuple) else (out,)) if o.requires_grad and o.numel()]
+    leaves = [a for a in args if isinstance(a, torch.Tensor) and a.requires_grad]
+    first = torch.autograd.grad(sum((o * o).sum() for o in outs), leaves, create_graph=True, allow_unused=True)
+    second = torch.autograd.grad(sum((g * g).sum() for g in first if g is not None), leaves, allow_unused=True)
+    return outs + [g for g in (*first, *second)], sorted(saved)
+
+
+@pytest.mark.parametrize("kind", ["conv", "dense", "norm", "irreps"])
+def test_operator_routes(kind):
+    """A plain call and the registered operator: the same values, derivatives and saved tensors (bit for bit:
+    the same kernels on the same inputs); vmap maps it, forward mode does the same and a tracer sees the operator."""
+    from torch.fx.experimental.proxy_tensor import make_fx
+    fn, args = _route_call(kind)
+    assert fn._direct(args)
+    got, saved = _route_results(fn, args)
+    want, want_saved = _route_results(fn.op, args)
+    assert saved == want_saved
+    for k, (a, b) in enumerate(zip(got, want)):
+        assert (a is None) == (b is None) and (a is None or torch.equal(a, b)), (kind, k)
+    with torch.no_grad():
+        a, b = fn(*args), fn.op(*args)
+    a, b = (a, b) if isinstance(a, tuple) else ((a,), (b,))
+    assert all(torch.equal(x, y) and not x.requires_grad for x, y in zip(a, b))
+
+    mapped = torch.func.vmap(lambda x: fn(x, *args[1:]))(args[0].detach()[None])
+    mapped = mapped if isinstance(mapped, tuple) else (mapped,)
+    assert all(torch.equal(x, y[0]) for x, y in zip(a, mapped))
+
+    def forward_mode(f):
+        fwd = torch.autograd.forward_ad
+        with fwd.dual_level():
+            try:
+                out = f(fwd.make_dual(args[0].detach(), torch.ones_like(args[0])), *args[1:])
+                return fwd.unpack_dual(out[0] if isinstance(out, tuple) else out).tangent is None
+            except RuntimeError as e:
+                return str(e)
+
+    assert forward_mode(fn) == forward_mode(fn.op)
+    graph = make_fx(lambda x: fn(x, *args[1:]))(args[0].detach())
+    assert any("flashcart" in str(n.target) for n in graph.graph.nodes)

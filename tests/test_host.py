@@ -327,3 +327,36 @@ def test_alias_as_flashcart():
         for k in [k for k in sys.modules if k == "flashcart" or k.startswith("flashcart.")]:
             del sys.modules[k]
         sys.modules.update(saved)
+
+
+def test_operator_arguments_that_need_the_registry():
+    """An Operator runs its implementation itself only for plain GPU tensors and arguments of the exact types;
+    everything else reaches the registered operator, which converts or refuses it."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    from flashcart_amd.o3 import _ops
+    x = torch.zeros(4, 3)
+    assert not _ops.irreps_fwd._direct((x, 2))  # not on a GPU
+    with FakeTensorMode(allow_non_fake_inputs=True):
+        f = torch.empty(4, 3, device="cuda")
+        assert f.is_cuda and not _ops.irreps_fwd._direct((f, 2))
+        assert _ops.irreps_fwd(f, 2).shape == (4, 9)
+    assert _ops._observed() is False
+
+    class Gpu(torch.Tensor):  # stands in for a GPU tensor
+        is_cuda = True
+
+    g = Gpu()
+    plain = _ops._EXACT["Tensor"]
+    sig = _ops.irreps_fwd.exact
+    assert sig[0] is plain and sig[1] == (int,)
+    op = _ops.Operator.__new__(_ops.Operator)
+    op.required, op.exact, op.items = 2, ((Gpu,), (int,), (list, tuple)), ((2, int),)
+    assert op._direct((g, 1)) and op._direct((g, 1, [1, 2])) and op._direct((g, 1, ()))
+    for bad in ((g,), (g, 1.0), (g, True), (g, 1, [1.0]), (g, 1, [], 0), (x, 1), (None, 1)):
+        assert not op._direct(bad), bad
+    for args in ((x,), (x, 1.5), (x, 2, 3), ("x", 2)):
+        with pytest.raises(Exception) as a:
+            _ops.irreps_fwd(*args)
+        with pytest.raises(Exception) as b:
+            _ops.irreps_fwd.op(*args)
+        assert type(a.value) is type(b.value)
