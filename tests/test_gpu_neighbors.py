@@ -102,3 +102,27 @@ def test_empty_and_single_atom():
     ei, sh = neighbor_pairs_device(torch.zeros(0, 3, dtype=torch.float64, device=DEV), np.eye(3) * 5, True, 3.0)
     assert ei.shape == (2, 0) and sh.shape == (0, 3)
     _same(np.array([[0.5, 0.5, 0.5]]), np.eye(3) * 2.0, True, 4.5, "one atom, its own images")
+
+
+@pytest.mark.parametrize("axis", [0, 1, 2])
+@pytest.mark.parametrize("thin,n", [(0.9, 5), (2.3, 20), (11.0, 200)])
+def test_runs_of_thin_cells(axis, thin, n):
+    """A cell thinner than the cutoff along one axis (up to 17 images of a column, more runs of candidates
+    than lanes) or a little wider than one bin, periodic there and open or periodic elsewhere."""
+    rng = np.random.default_rng(n)
+    size = np.full(3, 17.0)
+    size[axis] = thin
+    cell = np.diag(size) + rng.normal(scale=0.05, size=(3, 3))
+    pos = rng.uniform(-0.5, 1.5, size=(n, 3)) @ cell
+    for pbc in (True, [k == axis for k in range(3)], [k != (axis + 1) % 3 for k in range(3)]):
+        assert _same(pos, cell, pbc, 7.0, f"axis {axis}, {thin}, pbc {pbc}") > 0
+
+
+@pytest.mark.parametrize("n", [2, 3, 4095, 4096, 4097, 12289])
+def test_scan_tiles(n):
+    """Atom and bin counts around the tiles of the prefix sum, many bins empty."""
+    rng = np.random.default_rng(n)
+    side = (n / 0.02) ** (1.0 / 3.0)
+    pos = rng.uniform(0.0, side, size=(n, 3))
+    for pbc in (True, [True, False, True]):
+        _same(pos, np.eye(3) * side, pbc, 2.5, f"{n} atoms, pbc {pbc}")
