@@ -509,8 +509,8 @@ __global__ void __launch_bounds__(256, 2) tp_bwd_kernel(TPArgs g) {
 
 // Backward of the interaction-layer convolution (one in2 channel, unreduced outputs),
 // specialised at compile time: C channels (every lane active, operand offsets are
-// immediates), the weight and edge-attribute gradients always formed, the per-edge in1
-// messages when NEED1. Same arithmetic, in the same order, as tp_bwd_kernel<..., CONV, BC2>;
+// immediates), the per-edge in1 messages when NEED1, the weight gradient when NEEDW, the
+// edge-attribute gradient when NEED2 (there written only if asked for). Same arithmetic, in the same order, as tp_bwd_kernel<..., CONV, BC2>;
 // without the run-time flags the path contractions are one basic block, so loads, stores and
 // LDS reads of neighbouring paths interleave with their FMAs. The edge loop is unrolled by
 // two with two operand sets (no register copies between iterations): the operands of the
@@ -524,7 +524,7 @@ __host__ __device__ constexpr int bwd_conv_chunk() {
   return AmatLayout<L1, L2, LO, SYM>::chunk >= 2 ? (AmatLayout<L1, L2, LO, SYM>::chunk & ~1) : 2;
 }
 
-template <int L1, int L2, int LO, bool SYM, int C, int EG, bool NEED1>
+template <int L1, int L2, int LO, bool SYM, int C, int EG, bool NEED1, bool NEEDW, bool NEED2>
 __global__ void __launch_bounds__(C * EG, 2) tp_bwd_conv_kernel(TPArgs g) {
   using CF = TPConfig<L1, L2, LO, SYM>;
   using PL = typename CF::PL;
@@ -578,10 +578,10 @@ __global__ void __launch_bounds__(C * EG, 2) tp_bwd_conv_kernel(TPArgs g) {
   auto load_rows = [&](int64_t j, int64_t wrow, EdgeOps<D1, D2, NP>& o) {
     const float* xr = g.in1 + j * S1 + f;
 #pragma unroll
-    for (int u = 0; u < D1; ++u) o.x[u] = xr[u * C];
+    for (int u = 0; u < D1; ++u) o.x[u] = NEEDW || NEED2 ? xr[u * C] : 0.f;
     const float* wr = (wrow < 0 ? zero_weight_row : g.w + wrow * SW) + f;
 #pragma unroll
-    for (int i = 0; i < NP; ++i) o.w[i] = wr[i * C];
+    for (int i = 0; i < NP; ++i) o.w[i] = NEED1 || NEED2 ? wr[i * C] : 0.f;
   };
   // operands of edge e = (chunk q's first edge) + s, s < CH, from the staged indices
   auto load = [&](int64_t e, int q, int s, EdgeOps<D1, D2, NP>& o) {
@@ -596,7 +596,9 @@ __global__ void __launch_bounds__(C * EG, 2) tp_bwd_conv_kernel(TPArgs g) {
   // loaded register is first used, count conservatively across the loop's paths and waited for
   // the loads just issued.) A chunk boundary waits for everything: the coupling-matrix fill
   // waits for its own loads, issued after all others.
-  constexpr int LD = D1 + NP, ST = NP + (NEED1 ? D1 : 0);
+  // (in1 serves the weight and in2 gradients, the weights those of in1 and in2)
+  constexpr int LD = (NEEDW || NEED2 ? D1 : 0) + (NEED1 || NEED2 ? NP : 0);
+  constexpr int ST = (NEEDW ? NP : 0) + (NEED1 ? D1 : 0);
   constexpr int VM_STEP = LD + ST < 63 ? LD + ST : 63;  // at most 63 can be outstanding
   auto wait_operands = [&]() {
     vm_wait_barrier();
@@ -609,7 +611,7 @@ __global__ void __launch_bounds__(C * EG, 2) tp_bwd_conv_kernel(TPArgs g) {
     for (int u = 0; u < D1; ++u) gx[u] = 0.f;
 #pragma unroll
     for (int u = 0; u < R2; ++u) gy[u] = 0.f;
-    float* gwr = g.grad_w + e * SW + f;
+    float* gwr = NEEDW ? g.grad_w + e * SW + f : nullptr;
     static_for<NP>([&](auto ic) {
       constexpr int i = decltype(ic)::value;
       constexpr PathDesc P = PL::at(i);
@@ -622,22 +624,28 @@ __global__ void __launch_bounds__(C * EG, 2) tp_bwd_conv_kernel(TPArgs g) {
 #pragma unroll
       for (int b = 0; b < TP::N1; ++b) v[b] = 0.f;
       TP::apply_t(ae + AL::template off<i>(), gop, v);
-      float s = 0.f;
+      if constexpr (NEEDW) {
+        float s = 0.f;
 #pragma unroll
-      for (int b = 0; b < TP::N1; ++b) s = fmaf(v[b], xp[b], s);
-      gwr[i * C] = s;
+        for (int b = 0; b < TP::N1; ++b) s = fmaf(v[b], xp[b], s);
+        gwr[i * C] = s;
+      }
       if constexpr (NEED1) {
 #pragma unroll
         for (int b = 0; b < TP::N1; ++b) gx[P.r1 * P.r1 + b] = fmaf(cur.w[i], v[b], gx[P.r1 * P.r1 + b]);
       }
-      float xw[TP::N1];
+      if constexpr (NEED2) {
+        float xw[TP::N1];
 #pragma unroll
-      for (int b = 0; b < TP::N1; ++b) xw[b] = cur.w[i] * xp[b];
-      TP::vjp2(gop, xw, gy + P.r2 * P.r2);
+        for (int b = 0; b < TP::N1; ++b) xw[b] = cur.w[i] * xp[b];
+        TP::vjp2(gop, xw, gy + P.r2 * P.r2);
+      }
     });
-    const float s = wave_reduce_halving<R2, GW>(gy, lane);
-    const int v = (lane & (GW - 1)) >> SH2;
-    if ((lane & ((1 << SH2) - 1)) == 0 && v < D2) red_lds[(slot * NWG + wig) * D2 + v] = s;
+    if constexpr (NEED2) {
+      const float s = wave_reduce_halving<R2, GW>(gy, lane);
+      const int v = (lane & (GW - 1)) >> SH2;
+      if ((lane & ((1 << SH2) - 1)) == 0 && v < D2) red_lds[(slot * NWG + wig) * D2 + v] = s;
+    }
     if constexpr (NEED1) {
       float* mr = g.grad_in1 + e * S1 + f;
 #pragma unroll
@@ -695,7 +703,7 @@ __global__ void __launch_bounds__(C * EG, 2) tp_bwd_conv_kernel(TPArgs g) {
     if (n_next > 0) fill_amat<L1, L2, LO, SYM>(g.in2, c1, n_next, a_lds + (buf ^ 1) * CH * AL::total, lane, wave, NW);
     if (c1 + CH < e1) fill_idx(c1 + CH, q + 2);
     __syncthreads();
-    for (int k = t; k < n * D2; k += T) {
+    for (int k = NEED2 && g.grad_in2 ? t : n * D2; k < n * D2; k += T) {
       const int slot = k / D2, u = k % D2;
       float s = 0.f;
 #pragma unroll
@@ -1029,8 +1037,11 @@ bool launch_bwd_conv(const TPArgs& g, dim3 grid, hipStream_t stream) {
   if constexpr (bwd_conv_chunk<L1, L2, LO, SYM>() % (2 * EG) != 0) {
     return false;
   } else {
-    if (g.grad_in1) hipLaunchKernelGGL((tp_bwd_conv_kernel<L1, L2, LO, SYM, C, EG, true>), grid, dim3(C * EG), 0, stream, g);
-    else hipLaunchKernelGGL((tp_bwd_conv_kernel<L1, L2, LO, SYM, C, EG, false>), grid, dim3(C * EG), 0, stream, g);
+    const auto fn = !g.grad_w ? tp_bwd_conv_kernel<L1, L2, LO, SYM, C, EG, true, false, false>
+                    : g.grad_in1 ? tp_bwd_conv_kernel<L1, L2, LO, SYM, C, EG, true, true, true>
+                    : g.grad_in2 ? tp_bwd_conv_kernel<L1, L2, LO, SYM, C, EG, false, true, true>
+                                 : tp_bwd_conv_kernel<L1, L2, LO, SYM, C, EG, false, true, false>;
+    hipLaunchKernelGGL(fn, grid, dim3(C * EG), 0, stream, g);
     return true;
   }
 }
@@ -1098,8 +1109,14 @@ int launch_tp(const TPArgs& g, bool conv, bool bwd, hipStream_t stream) {
       return kSendNotApplicable;
     }
     if constexpr (!SYM && L2 >= 1) {
-      // interaction-layer shape: the compile-time specialisation
-      if (conv && bc2 && !g.reduced && !g.shared_w && g.grad_w && g.grad_in2 && g.F1 == g.C &&
+      // interaction-layer shape: the compile-time specialisation, for the weight gradient with any others and
+      // for the in1 gradient alone (a second derivative asks for these; in1 and in2 without the weights would
+      // need a kernel that measured 122 registers spilled). 2x3->3 product, 4,000 receivers of 20 edges, general
+      // kernel / specialised: weight gradient alone 382 / 53 us with 32 channels, 391 / 112 with 64, 467 / 203
+      // with 128; in1 alone 382 / 86, 409 / 156, 486 / 321; in1 and weights 411 / 132, 453 / 246, 615 / 482.
+      // 48 receivers, weight gradient: 69 / 27, 68 / 26, 69 / 24 us
+      if (conv && bc2 && !g.reduced && !g.shared_w && (g.grad_w || (g.grad_in1 && !g.grad_in2)) &&
+          g.F1 == g.C &&
           (g.C == 32 || g.C == 64 || g.C == 128)) {  // per-edge weights: the kernel reads w[e] rows
         bool done = false;
         if (g.C == 128) {

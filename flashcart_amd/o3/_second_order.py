@@ -60,16 +60,6 @@ def _tp_bwd_setup(ctx, inputs, output):
     ctx.computed = (bool(n1), bool(n2), bool(nw))
 
 
-def _conv_bwd_specialised(cfg, conv: bool) -> bool:
-    """Whether fc_tp_bwd runs a convolution of this configuration on its compile-time
-    specialised kernel when the weight and in2 gradients are both requested: per-edge
-    weights, one in2 channel, unreduced outputs, 32, 64 or 128 in1 channels, in2 rank >= 1,
-    no symmetric product (the launcher's conditions in csrc/fc_tp_impl.h)."""
-    l1, l2, lo, f1, f2, sym, shared = cfg[:7]
-    red = cfg[12]
-    return conv and not shared and not red and not sym and f2 == 1 and f1 in (32, 64, 128) and l2 >= 1
-
-
 def _tp_dbwd(ctx, c1, c2, cw):
     """Backward of tp_bwd (reference tp_dbwd, src/flashcart/o3/_tensor_product.py:789-1093)."""
     go, in1, in2, w, ii, jj, rp, sp, sq, adiv = ctx.saved_tensors
@@ -99,11 +89,7 @@ def _tp_dbwd(ctx, c1, c2, cw):
                  and t[2] is not None]
         d_go = _acc(*[fwd(*t) for t in terms]) if terms else None
     a = bwd(c1, in2, w, False, need[2], need[3]) if c1 is not None else (None,) * 3
-    # the in2 gradient of the second product is not needed; asking for it anyway lets an
-    # interaction-layer convolution take the kernel specialised for (in1, in2, weight) gradients
-    b = bwd(in1, c2, w, need[1], _conv_bwd_specialised(cfg, ii is not None) and bool(need[3]), need[3]) \
-        if c2 is not None else (None,) * 3
-    b = (b[0], None, b[2])
+    b = bwd(in1, c2, w, need[1], False, need[3]) if c2 is not None else (None,) * 3
     c = bwd(in1, in2, cw, need[1], need[2], False) if cw is not None else (None,) * 3
     d_in1 = _acc(b[0], c[0]) if need[1] else None
     d_in2 = _acc(a[1], c[1]) if need[2] else None

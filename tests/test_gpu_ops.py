@@ -893,3 +893,35 @@ def test_operator_routes(kind):
     assert forward_mode(fn) == forward_mode(fn.op)
     graph = make_fx(lambda x: fn(x, *args[1:]))(args[0].detach())
     assert any("flashcart" in str(n.target) for n in graph.graph.nodes)
+
+
+@pytest.mark.parametrize("C", [32, 64, 128])
+@pytest.mark.parametrize("l1,l2,lo", [(2, 3, 3), (0, 2, 2), (3, 3, 3)])
+@pytest.mark.parametrize("degrees", [(1, 0, 2, 33, 66), (17, 16, 15) * 255])
+def test_tp_conv_some_gradients(C, l1, l2, lo, degrees):
+    """A convolution's backward asked for each subset of its gradients (other kernels for some subsets):
+    the gradients of the full request up to its sums' rounding, and empty tensors for the rest."""
+    ops = _ops()
+    from flashcart_amd.o3._graph import build_graph
+    ei = random_csr_graph(len(degrees), degrees, seed=C, allow_self=True)
+    graph = build_graph(ei.to(DEV), len(degrees))
+    g = torch.Generator(device=DEV).manual_seed(C + l1)
+    meta = ops.tp_meta(l1, l2, lo, C, 1, False, False)
+    n, e = len(degrees), ei.shape[1]
+    in1, in2, w, go = (torch.randn(*s, device=DEV, generator=g) for s in (
+        (n, (l1 + 1) ** 2 * C), (e, (l2 + 1) ** 2), (e, meta[-1] * C), (n, sum(meta[2]))))
+
+    def run(*need):
+        return ops.tp_bwd(go, in1, in2, w, graph.idx_i, graph.idx_j, l1, l2, lo, C, 1, False, False, *meta, False,
+                          *need, graph.rowptr, graph.sender_perm, graph.sender_ptr, 0.7)
+
+    # each gradient's terms in absolute value: the full request of the absolute operands bounds nothing (signed
+    # coupling constants), so the bound is relative to the largest entry, as for the other products here
+    want = run(True, True, True)
+    for mask in range(1, 8):
+        need = [bool(mask & b) for b in (1, 2, 4)]
+        for k, (a, b, on) in enumerate(zip(run(*need), want, need)):
+            if on:
+                _close(a, b, f"gradient {k} of {need}")
+            else:
+                assert a.numel() == 0
