@@ -353,7 +353,9 @@ def _cpu_rate(fn, units, budget_s=8.0):
     return units * calls / dt, cores, calls, dt
 
 
-MFMA_PEAK_TFLOPS = 157.3  # MI355X dense fp32 MFMA
+# MI355X dense fp32 MFMA: the rate the float32 matrix instructions could reach. Most of the maps form their float32
+# products from six bf16 products each, whose own ceiling is 2,500 / 6 = 417 TFLOP/s.
+MFMA_PEAK_TFLOPS = 157.3
 
 
 def mfma_in_step(step, dev, launches=None):
