@@ -484,7 +484,9 @@ static int64_t nl_build(int64_t n, const double* pos, const double* cell, const 
   }
   const int64_t nbins = (int64_t)p.nb[0] * p.nb[1] * p.nb[2];
   p.ns2 = p.pbc[2] ? (2 * p.D[2] + p.nb[2] - 1) / p.nb[2] + 1 : 1;
-  // Columns of bins beyond 31 bits (a cell thousands of times thinner than the cutoff): the host list's.
+  // A cell a million times thinner than the cutoff, or columns of bins beyond 31 bits: the host list's.
+  for (int k = 0; k < 3; ++k)
+    if (p.D[k] < 0 || p.D[k] > (1 << 20)) return -FC_ERR_SHAPE;
   if ((2.0 * p.D[0] + 1.0) * (2.0 * p.D[1] + 1.0) * p.ns2 > 2147483647.0) return -FC_ERR_SHAPE;
   int32_t* const status = ws.status->status;
   hipLaunchKernelGGL(nl_init_kernel, dim3((unsigned)((nbins + bs - 1) / bs)), dim3(bs), 0, s, nbins, ws.hist, status);

@@ -205,8 +205,10 @@ class Operator:
                            if q.annotation in _EXACT_ITEM)
         functools.update_wrapper(self, impl)
 
-    def register_fake(self, fn):
-        return self.op.register_fake(fn)
+    def __getattr__(self, name):  # whatever else a registered operator offers
+        if name == "op":
+            raise AttributeError(name)
+        return getattr(self.op, name)
 
     def register_autograd(self, backward, setup_context):
         self.op.register_autograd(backward, setup_context=setup_context)

@@ -126,3 +126,21 @@ def test_scan_tiles(n):
     pos = rng.uniform(0.0, side, size=(n, 3))
     for pbc in (True, [True, False, True]):
         _same(pos, np.eye(3) * side, pbc, 2.5, f"{n} atoms, pbc {pbc}")
+
+
+@pytest.mark.parametrize("spacing", [1e-10, 1e-4])
+def test_cells_beyond_the_device_list(spacing):
+    """Cells thinner than the device list has room for (bins counted in 32 bits; more than 1,024 pairs) are
+    refused before or after the search, as sizes for the host list."""
+    from flashcart_amd import _lib
+    from flashcart_amd.data.neighbors import host_fallback_needed
+    lib = _lib.load()
+    pos = torch.zeros(2, 3, dtype=torch.float64, device=DEV)
+    cell = np.diag([8.0, spacing, 9.0])
+    flags = np.ones(3, dtype=np.int32)
+    ws = torch.empty(int(lib.fc_neighbor_list_device_workspace(2)), dtype=torch.uint8, device=DEV)
+    out = torch.empty(2, 64, dtype=torch.int64, device=DEV)
+    sh = torch.empty(64, 3, dtype=torch.int32, device=DEV)
+    n = lib.fc_neighbor_list_device(2, pos.data_ptr(), cell.ctypes.data, flags.ctypes.data, 4.0, 64, out[0].data_ptr(),
+                                    out[1].data_ptr(), sh.data_ptr(), ws.data_ptr(), ws.numel(), _lib.stream_of(pos))
+    assert host_fallback_needed(n)
