@@ -215,6 +215,7 @@ def require_device(name: str, t: torch.Tensor, dtype: torch.dtype = torch.float3
 
 def contig(name: str, t: torch.Tensor, dtype: torch.dtype = torch.float32) -> torch.Tensor:
     require_device(name, t, dtype)
+    t = t.resolve_neg()  # (a negated view's memory holds the values before negation)
     return t if t.is_contiguous() else t.contiguous()
 
 

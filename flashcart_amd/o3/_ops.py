@@ -189,9 +189,9 @@ class Operator:
     implementation, under an ``autograd.Function`` of the same formula where a gradient is wanted, without
     the operator registry's argument handling, which costs more host time (100 us for the 24 arguments of
     ``tp_fwd``) than the kernels of a small call take. Anything that has to see or rewrite the operator itself
-    (``_observed``, tensor subclasses, tensors that are not on a GPU) and every call that the registry would
-    convert or refuse (keywords, arguments of other types or counts) goes through the registered operator;
-    both run the same implementation and the same backward."""
+    (``_observed``, tensor subclasses, tensors that are not on a GPU or whose memory does not hold their values,
+    as a negated view's) and every call that the registry would convert or refuse (keywords, arguments of other
+    types or counts) goes through the registered operator; both run the same implementation and the same backward."""
 
     def __init__(self, name: str, impl):
         self.op = torch.library.custom_op(name, mutates_args=())(impl)
@@ -233,7 +233,10 @@ class Operator:
         if not self.required <= len(args) <= len(self.exact):
             return False
         for a, exact in zip(args, self.exact):
-            if type(a) not in exact or (exact[0] is Tensor and a is not None and not a.is_cuda):
+            if type(a) not in exact:
+                return False
+            # (the dispatcher writes out negated views and zero tensors before it calls the implementation)
+            if isinstance(a, Tensor) and (not a.is_cuda or a.is_neg() or a._is_zerotensor()):
                 return False
         return all(type(x) is item for k, item in self.items if k < len(args) for x in args[k])
 

@@ -895,6 +895,94 @@ def test_operator_routes(kind):
     assert any("flashcart" in str(n.target) for n in graph.graph.nodes)
 
 
+def _operator_call(name):
+    """Arguments of a small call of an operator, the differentiable ones leaves that require gradients (none for the
+    operators without a formula of their own)."""
+    ops = _ops()
+    from flashcart_amd import _lib
+    gen = torch.Generator().manual_seed(29)
+    grads = getattr(ops, name).function is not None
+
+    def t(*shape, low=None):
+        v = torch.randn(*shape, generator=gen) if low is None else torch.rand(*shape, generator=gen) + low
+        return v.to(DEV).requires_grad_(grads)
+
+    i, j = (v.to(DEV).int() for v in random_csr_graph(9, [4, 0, 3], seed=3))
+    e, radial = i.numel(), (_lib.BASIS_BESSEL, 8, 0.0, 5.0, 6)
+    unit = unit_vectors(17, seed=2).float().to(DEV).requires_grad_(grads)
+    meta = ops.tp_meta(1, 1, 1, 8, 1, False, False)
+    conv = (t(9, 32), t(e, 4), t(e, 8 * meta[-1]), i, j, 1, 1, 1, 8, 1, False, False, *meta)
+    maps = (t(12, 8), t(12, 8), None, None, None, 1, 1, 8, 12, [1, 1], [0.3, 0.2], 0.7)
+    edges = (t(9, 3), t(e, 3), i, j, None, None, None, None, 2, *radial)
+    mlp = (t(13, 8), t(64, 8), 0.3, t(64, 64), 0.2)
+    return {
+        "irreps_fwd": lambda: (unit, 2),
+        "irreps_bwd": lambda: (t(17, 9), unit, 2),
+        "irreps_dbwd": lambda: (t(17, 9), unit, t(17, 3), 2),
+        "radial_fwd": lambda: (t(17, low=0.5), *radial),
+        "radial_bwd": lambda: (t(17, low=0.5), t(17, 8), t(17), *radial),
+        "edge_geometry": lambda: edges,
+        "edge_geometry_bwd": lambda: (t(e, 9), t(e, 8), t(e), *edges, True),
+        "tp_fwd": lambda: conv,
+        "tp_bwd": lambda: (t(9, sum(meta[2])), *conv, False, True, True, True),
+        "linear_fwd_op": lambda: (t(13, 32), *maps, t(13, 48)),
+        "linear_bwd_op": lambda: (t(13, 48), *maps, t(13, 32)),
+        "dense_fwd": lambda: (t(13, 8), t(16, 8), t(16), 0.3, 1),
+        "dense_bwd": lambda: (t(13, 16), t(13, 16), t(16, 8), 0.3, 1),
+        "radial_mlp_fwd": lambda: (*mlp, t(40, 64), 0.1),
+        "radial_mlp_bwd": lambda: (t(13, 64), *mlp),
+        "segment_sum": lambda: (t(13, 4), torch.tensor([0, 5, 5, 13], dtype=torch.int32, device=DEV),
+                                torch.tensor([0] * 5 + [2] * 8, dtype=torch.int32, device=DEV)),
+        "rms_norm": lambda: (t(7, 72), t(3, 8), 2, 1e-5),
+        "rms_norm_bwd": lambda: (t(7, 72), t(7, 72), t(3, 8), t(7, low=0.5), 2),
+        "gate": lambda: (t(7, 72), t(7, 24), 2, 1),
+        "gate_bwd": lambda: (t(7, 72), t(7, 72), t(7, 24), 2, 1, True, True),
+    }[name]()
+
+
+def _operator_names():
+    ops = _ops()
+    return sorted(k for k, v in vars(ops).items() if isinstance(v, ops.Operator))
+
+
+def _values_and_gradients(fn, args, leaves):
+    """Outputs of a call and their gradients by ``leaves`` (a fixed cotangent)."""
+    out = fn(*args)
+    outs = [o for o in (out if isinstance(out, tuple) else (out,)) if o.numel()]
+    diff = [o for o in outs if o.requires_grad]
+    if not leaves:
+        assert not diff
+        return outs, []
+    return outs, torch.autograd.grad(sum((o * (1.0 + o.detach())).sum() for o in diff), leaves, allow_unused=True)
+
+
+@pytest.mark.parametrize("name", _operator_names())
+def test_every_operator_route(name):
+    """Every operator called plainly, through the registry, and with negated views for its floating-point arguments:
+    the same values and gradients, bit for bit. The profiler sees the operator."""
+    fn = getattr(_ops(), name)
+    args = _operator_call(name)
+    assert fn._direct(args)
+    leaves = [a for a in args if isinstance(a, torch.Tensor) and a.requires_grad]
+    got, grads = _values_and_gradients(fn, args, leaves)
+    want, want_grads = _values_and_gradients(fn.op, args, leaves)
+    assert len(got) == len(want) and all(torch.equal(a, b) for a, b in zip(got, want))
+    assert all((a is None) == (b is None) and (a is None or torch.equal(a, b)) for a, b in zip(grads, want_grads))
+
+    # the same values behind a negation: every floating-point argument, also a single element
+    bases = [(-a.detach()).requires_grad_(a.requires_grad) if isinstance(a, torch.Tensor) and a.is_floating_point()
+             else a for a in args]
+    views = [torch._neg_view(b) if isinstance(b, torch.Tensor) and b.is_floating_point() else b for b in bases]
+    neg, neg_grads = _values_and_gradients(
+        fn, views, [b for b in bases if isinstance(b, torch.Tensor) and b.requires_grad])
+    assert all(torch.equal(a, b) for a, b in zip(neg, want))
+    assert all((a is None) == (b is None) and (a is None or torch.equal(a, -b)) for a, b in zip(neg_grads, want_grads))
+
+    with torch.no_grad(), torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]) as prof:
+        fn(*args)
+    assert any(ev.key.startswith("flashcart::") for ev in prof.key_averages())
+
+
 @pytest.mark.parametrize("C", [32, 64, 128])
 @pytest.mark.parametrize("l1,l2,lo", [(2, 3, 3), (0, 2, 2), (3, 3, 3)])
 @pytest.mark.parametrize("degrees", [(1, 0, 2, 33, 66), (17, 16, 15) * 255])

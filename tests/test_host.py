@@ -360,3 +360,35 @@ def test_operator_arguments_that_need_the_registry():
         with pytest.raises(Exception) as b:
             _ops.irreps_fwd.op(*args)
         assert type(a.value) is type(b.value)
+
+
+def test_operator_lazy_values_need_the_registry():
+    """A tensor whose memory does not hold its values yet (a negated view, of one element also when contiguous; a
+    zero tensor without memory) goes through the registered operator, which writes them out for the implementation.
+    The condition is the same for every operator, so it is checked on each with stand-ins for GPU tensors."""
+    from flashcart_amd.o3 import _ops
+
+    class Gpu(torch.Tensor):
+        is_cuda = True
+
+    def stand_in(t):
+        return t.as_subclass(Gpu)
+
+    negated = torch.tensor([0.3 + 0.77j]).conj().imag
+    assert negated.is_neg() and negated.is_contiguous()
+    zero = torch._efficientzerotensor(1, 3)
+    assert zero.data_ptr() == 0
+    operators = [op for op in vars(_ops).values() if isinstance(op, _ops.Operator)]
+    assert len(operators) >= 20
+    for op in operators:
+        exact = tuple((Gpu,) if e is _ops._EXACT["Tensor"] else (Gpu, type(None)) if Gpu not in e and e[0] is torch.Tensor
+                      else e for e in op.exact)
+        probe = _ops.Operator.__new__(_ops.Operator)
+        probe.required, probe.exact, probe.items = op.required, exact, op.items
+        value = {int: 1, bool: True, float: 1.0, list: []}
+        args = [stand_in(torch.ones(1)) if e[0] is Gpu else value[e[0]] for e in exact]
+        assert probe._direct(args), op
+        for k, e in enumerate(exact):
+            if e[0] is Gpu:
+                for lazy in (negated, torch._neg_view(torch.ones(4)), zero):
+                    assert not probe._direct(args[:k] + [stand_in(lazy)] + args[k + 1:]), (op, k)
