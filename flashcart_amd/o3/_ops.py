@@ -184,17 +184,21 @@ def _observed() -> bool:
                 or getattr(torch.autograd.forward_ad, "_current_level", 0) >= 0)
 
 
-class Operator:
-    """A registered operator (``torch.ops.flashcart.*``) and its Python callable. Calling it runs the
-    implementation, under an ``autograd.Function`` of the same formula where a gradient is wanted, without
-    the operator registry's argument handling, which costs more host time (100 us for the 24 arguments of
-    ``tp_fwd``) than the kernels of a small call take. Anything that has to see or rewrite the operator itself
-    (``_observed``, tensor subclasses, tensors that are not on a GPU or whose memory does not hold their values,
-    as a negated view's) and every call that the registry would convert or refuse (keywords, arguments of other
-    types or counts) goes through the registered operator; both run the same implementation and the same backward."""
+class Operator(torch.library.CustomOpDef):
+    """A registered operator (``torch.ops.flashcart.*``). Calling it runs the implementation, under an
+    ``autograd.Function`` of the same formula where a gradient is wanted, without the operator registry's
+    argument handling, which costs more host time (100 us for the 24 arguments of ``tp_fwd``) than the kernels
+    of a small call take. Anything that has to see or rewrite the operator itself (``_observed``, tensor
+    subclasses, tensors that are not on a GPU or whose memory does not hold their values, as a negated view's)
+    and every call that the registry would convert or refuse (keywords, arguments of other types or counts)
+    goes through the registered operator ``op``; both run the same implementation and the same backward."""
 
-    def __init__(self, name: str, impl):
-        self.op = torch.library.custom_op(name, mutates_args=())(impl)
+    @classmethod
+    def register(cls, name: str, impl) -> "Operator":
+        self = torch.library.custom_op(name, mutates_args=())(impl)
+        self.__class__ = cls  # the same object and registrations, called otherwise
+        namespace, short = name.split("::")
+        self.op = getattr(getattr(torch.ops, namespace), short).default
         self.impl = impl
         self.function = None
         params = tuple(inspect.signature(impl).parameters.values())
@@ -204,21 +208,18 @@ class Operator:
         self.items = tuple((k, _EXACT_ITEM[q.annotation]) for k, q in enumerate(params)
                            if q.annotation in _EXACT_ITEM)
         functools.update_wrapper(self, impl)
+        return self
 
-    def __getattr__(self, name):  # whatever else a registered operator offers
-        if name == "op":
-            raise AttributeError(name)
-        return getattr(self.op, name)
-
-    def register_autograd(self, backward, setup_context):
-        self.op.register_autograd(backward, setup_context=setup_context)
+    def register_autograd(self, backward, /, *, setup_context=None):
+        super().register_autograd(backward, setup_context=setup_context)
         impl = self.impl
 
         class Direct(torch.autograd.Function):
             @staticmethod
             def forward(ctx, *inputs):
                 output = impl(*inputs)
-                setup_context(ctx, inputs, output)
+                if setup_context is not None:
+                    setup_context(ctx=ctx, inputs=inputs, output=output)
                 return output
 
             @staticmethod
@@ -253,7 +254,7 @@ class Operator:
 
 def operator(name: str):
     """Register the decorated implementation as ``torch.ops.flashcart.<name>``."""
-    return lambda impl: Operator(name, impl)
+    return lambda impl: Operator.register(name, impl)
 
 
 def _register_autograd(op, backward, setup_context) -> None:

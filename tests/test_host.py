@@ -392,3 +392,46 @@ def test_operator_lazy_values_need_the_registry():
             if e[0] is Gpu:
                 for lazy in (negated, torch._neg_view(torch.ones(4)), zero):
                     assert not probe._direct(args[:k] + [stand_in(lazy)] + args[k + 1:]), (op, k)
+
+
+Tensor = torch.Tensor  # (operators' annotations are read as text)
+
+
+def _scratch_operator(name):
+    """An operator for one test, x -> 2 x, whose calls count as plain ones on the CPU."""
+    from flashcart_amd.o3 import _ops
+
+    def double(x: "Tensor") -> "Tensor":
+        return 2 * x
+
+    op = _ops.Operator.register(f"flashcart_test::{name}", double)
+    op.register_fake(torch.empty_like)
+    op._direct = lambda args: True
+    return op
+
+
+def test_operators_are_registered_operators():
+    """torch.library's functions that take an operator take the callables of this package, by object and by name, and
+    compilers see the operator itself in a whole graph."""
+    from flashcart_amd.o3 import _ops
+    op = _ops.irreps_fwd
+    assert isinstance(op, torch.library.CustomOpDef)
+    x = torch.zeros(4, 3)
+    # (no kernel for the CPU: the checks that run the operator end in its own error)
+    with pytest.raises(Exception, match="ROCm devices only"):
+        torch.library.opcheck(op, (x, 2), test_utils="test_schema")
+    torch.library.opcheck(op, (x, 2), test_utils="test_autograd_registration")
+    for k, by_name in enumerate((False, True)):
+        own = _scratch_operator(f"vmap{k}")
+        torch.library.register_vmap(f"flashcart_test::vmap{k}" if by_name else own,
+                                    lambda info, in_dims, x: (x + 1, in_dims[0]))
+        assert torch.equal(torch.func.vmap(own)(x), x + 1)
+    assert _ops.irreps_fwd.__name__ == "irreps_fwd" and "irreps_bwd" in repr(_ops.irreps_bwd)
+    seen = []
+
+    def backend(graph, inputs):
+        seen.extend(str(n.target) for n in graph.graph.nodes if n.op == "call_function")
+        return lambda *a: (x.new_zeros(4, 9),)
+
+    out = torch.compile(lambda v: op(v, 2), backend=backend, fullgraph=True)(x)
+    assert out.shape == (4, 9) and any("flashcart.irreps_fwd" in t for t in seen)
