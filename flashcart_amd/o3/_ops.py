@@ -176,6 +176,10 @@ _EXACT = {"Tensor": _PLAIN, "Optional[Tensor]": _PLAIN + (type(None),), "int": (
 _EXACT_ITEM = {"List[int]": int, "List[float]": float}
 
 
+# "namespace/operator/dispatch key" of the kernels that libraries of Python programs have put in
+_IMPLS = getattr(torch.library, "_impls", frozenset())
+
+
 def _observed() -> bool:
     if torch.compiler.is_compiling() or None in _QUERIES:
         return True
@@ -191,7 +195,10 @@ class Operator(torch.library.CustomOpDef):
     of a small call take. Anything that has to see or rewrite the operator itself (``_observed``, tensor
     subclasses, tensors that are not on a GPU or whose memory does not hold their values, as a negated view's)
     and every call that the registry would convert or refuse (keywords, arguments of other types or counts)
-    goes through the registered operator ``op``; both run the same implementation and the same backward."""
+    goes through the registered operator ``op``; both run the same implementation and the same backward. Once
+    somebody registers a kernel or an autocast rule of their own for it, every call goes there."""
+
+    overridden = False
 
     @classmethod
     def register(cls, name: str, impl) -> "Operator":
@@ -199,6 +206,7 @@ class Operator(torch.library.CustomOpDef):
         self.__class__ = cls  # the same object and registrations, called otherwise
         namespace, short = name.split("::")
         self.op = getattr(getattr(torch.ops, namespace), short).default
+        self.kernels = tuple(f"{namespace}/{short}/{key}" for key in ("CUDA", "AutogradCUDA", "AutocastCUDA"))
         self.impl = impl
         self.function = None
         params = tuple(inspect.signature(impl).parameters.values())
@@ -209,6 +217,14 @@ class Operator(torch.library.CustomOpDef):
                            if q.annotation in _EXACT_ITEM)
         functools.update_wrapper(self, impl)
         return self
+
+    def register_kernel(self, device_types, fn=None, /):
+        self.overridden = True
+        return super().register_kernel(device_types, fn)
+
+    def register_autocast(self, device_type, cast_inputs):
+        self.overridden = True
+        return super().register_autocast(device_type, cast_inputs)
 
     def register_autograd(self, backward, /, *, setup_context=None):
         super().register_autograd(backward, setup_context=setup_context)
@@ -242,7 +258,8 @@ class Operator(torch.library.CustomOpDef):
         return all(type(x) is item for k, item in self.items if k < len(args) for x in args[k])
 
     def __call__(self, *args, **kwargs):
-        if kwargs or _observed() or not self._direct(args):
+        if (kwargs or self.overridden or not _IMPLS.isdisjoint(self.kernels) or _observed()
+                or not self._direct(args)):
             return self.op(*args, **kwargs)
         args += self.defaults[len(args):]
         if torch.is_grad_enabled() and any(isinstance(a, Tensor) and a.requires_grad for a in args):

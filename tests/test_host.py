@@ -435,3 +435,42 @@ def test_operators_are_registered_operators():
 
     out = torch.compile(lambda v: op(v, 2), backend=backend, fullgraph=True)(x)
     assert out.shape == (4, 9) and any("flashcart.irreps_fwd" in t for t in seen)
+
+
+@pytest.mark.parametrize("by_name", [False, True])
+def test_operator_kernel_overrides(by_name):
+    """A kernel or an autocast rule registered for an operator is what a plain call runs from then on, and a kernel
+    switched off leaves the implementation."""
+    name = f"override_{'name' if by_name else 'object'}"
+    op = _scratch_operator(name)
+    op.register_autograd(lambda ctx, g: 2 * g)
+    target = f"flashcart_test::{name}" if by_name else op
+    x = torch.ones(3, requires_grad=True)
+
+    def gradient():
+        return torch.autograd.grad(op(x).sum(), x)[0]
+
+    assert torch.equal(op(x), 2 * x) and type(op(x).grad_fn).__name__ == "DirectBackward"
+    if by_name:
+        torch.library.register_kernel(target, "cpu", lambda x: 5 * x.detach())
+    else:
+        op.register_kernel("cpu")(lambda x: 5 * x.detach())
+    assert torch.equal(op(x), 5 * x) and torch.equal(gradient(), torch.full((3,), 2.0))
+    with op.set_kernel_enabled("cpu", enabled=False):
+        assert torch.equal(op(x), 2 * x)
+    assert torch.equal(op(x), 5 * x)
+
+    cast = _scratch_operator(name + "_cast")
+    torch.library.register_autocast(f"flashcart_test::{name}_cast" if by_name else cast, "cpu", torch.bfloat16)
+    with torch.autocast("cpu", torch.bfloat16):
+        assert cast(torch.ones(3)).dtype == torch.bfloat16
+    assert cast(torch.ones(3)).dtype == torch.float32
+
+    for key in ("CUDA", "AutogradCUDA", "AutocastCUDA"):  # a dispatcher kernel of another library
+        own = _scratch_operator(f"{name}_{key}")
+        assert own.kernels[0] == f"flashcart_test/{name}_{key}/CUDA"
+        own.op = lambda x: "registry"
+        lib = torch.library.Library("flashcart_test", "IMPL")
+        assert torch.equal(own(x.detach()), 2 * x)
+        lib.impl(f"{name}_{key}", lambda x: 7 * x, key)
+        assert own(x.detach()) == "registry"
