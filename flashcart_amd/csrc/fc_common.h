@@ -113,6 +113,19 @@ __device__ __forceinline__ int64_t xcd_row(int64_t n) {
   return (b % 8) * per + b / 8;
 }
 
+// Compute units of the current device.
+inline int device_cu_count() {
+  static int cus[64] = {0};
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+  if (cus[dev] <= 0) {
+    int v = 0;
+    if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || v <= 0) v = 256;
+    cus[dev] = v;
+  }
+  return cus[dev];
+}
+
 // Wave64 sum reduction (result valid in every lane).
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll

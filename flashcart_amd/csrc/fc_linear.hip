@@ -653,18 +653,6 @@ __global__ void __launch_bounds__(256, 2) gemm_pairsum_kernel(GemmBatch gb) {
   }
 }
 
-static int device_cu_count() {
-  static int cus[64] = {0};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  if (cus[dev] <= 0) {
-    int v = 0;
-    if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || v <= 0) v = 256;
-    cus[dev] = v;
-  }
-  return cus[dev];
-}
-
 // Whether gemm_split_kernel takes the batch.
 static bool split_ok(const GemmBatch& gb, int n_ranks) {
   if (gb.act || gb.act_bwd) return false;

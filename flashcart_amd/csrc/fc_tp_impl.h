@@ -1019,10 +1019,7 @@ constexpr bool wide_groups() {
 inline int conv_edge_groups(int64_t n_rows, int64_t n_edges, int C) {
   // 512 receivers x 8 edges with 32 channels: 29.0 us per forward + backward with four groups,
   // 32.4 us with eight (measured on the standalone product of the benchmark's first configuration)
-  // 128 channels, 42 edges a receiver, 2x3->3 product, forward / backward op: 32 receivers 69 / 156 us with one
-  // group, 39 / 66 us with four; 256: 77 / 181 and 37 / 87; 512: 87 / 197 and 60 / 165; 768: 95 / 238 and
-  // 88 / 240; 1,024: 109 / 299 and 120 / 319
-  if (C == 128) return n_rows < 768 && 8 * n_rows <= n_edges ? 4 : 1;
+  if (C == 128) return 8 * n_rows <= n_edges ? 4 : 1;  // and as wide_round allows
   const int max_eg = C == 32 || C == 64 ? 4 : 1;
   int eg = C == 32 ? 2 : 1;
   const double deg = n_rows > 0 ? (double)n_edges / (double)n_rows : 0.0;
@@ -1030,18 +1027,51 @@ inline int conv_edge_groups(int64_t n_rows, int64_t n_edges, int C) {
   return eg;
 }
 
+// Workgroups of a kernel that one CU holds (at least 1).
+inline int workgroups_per_cu(const void* kernel, int threads, size_t lds) {
+  int n = 0;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, threads, lds) != hipSuccess) n = 1;
+  return n < 1 ? 1 : n;
+}
+
+// Whether a 128-channel convolution of n_rows receivers runs on four edge groups, per_cu workgroups of which fit a
+// CU: as long as all of them run at once, up to three to a CU (more receivers were not measured). A second round is
+// begun only where the kernel fits a CU once and its receivers have second_degree edges or more. All 47 products of
+// wide_groups with 8, 16 and 42 edges a receiver, one group / four, forward and backward, in microseconds:
+//   2x3->3 (one to a CU)   32 receivers of 42 edges 48 / 21, 116 / 52; 257 of 8: 17 / 20, 34 / 33; 512 of 8: 19 / 25, 38 / 40;
+//                          512 of 42: 65 / 52, 157 / 144; 640 of 42: 66 / 70, 179 / 195
+//   2x2->2 (two forward)   512 of 8: 11.2 / 11.1; 512 of 42: 37 / 29; 640 of 8: 12 / 16; 640 of 42: 37 / 39
+//   1x1->1 (three or four) 767 of 8: 6.0 / 5.5, 16.8 / 16.6; 767 of 42: 25 / 16, 52 / 52
+inline bool wide_round(int per_cu, int64_t n_rows, int64_t n_edges, int second_degree) {
+  const int64_t cus = device_cu_count();
+  if (n_rows <= (per_cu < 3 ? per_cu : 3) * cus) return true;
+  return n_rows <= 2 * cus && n_edges >= second_degree * n_rows;
+}
+
 // The specialised convolution backward with C channels and EG edge groups; false (nothing
-// launched) when a full coupling-matrix chunk would not split evenly over the groups.
+// launched) when a full coupling-matrix chunk would not split evenly over the groups or, with 128
+// channels, wide_round is against them (16 edges a receiver for a second round: with 512 receivers the time of
+// one group over that of four is 0.98 to 1.15 with 16 edges and 0.89 to 1.04 with 8, in the products that fit once).
 template <int L1, int L2, int LO, bool SYM, int C, int EG>
 bool launch_bwd_conv(const TPArgs& g, dim3 grid, hipStream_t stream) {
   if constexpr (bwd_conv_chunk<L1, L2, LO, SYM>() % (2 * EG) != 0) {
     return false;
   } else {
-    const auto fn = !g.grad_w ? tp_bwd_conv_kernel<L1, L2, LO, SYM, C, EG, true, false, false>
-                    : g.grad_in1 ? tp_bwd_conv_kernel<L1, L2, LO, SYM, C, EG, true, true, true>
-                    : g.grad_in2 ? tp_bwd_conv_kernel<L1, L2, LO, SYM, C, EG, false, true, true>
-                                 : tp_bwd_conv_kernel<L1, L2, LO, SYM, C, EG, false, true, false>;
-    hipLaunchKernelGGL(fn, grid, dim3(C * EG), 0, stream, g);
+    constexpr void (*kernels[4])(TPArgs) = {tp_bwd_conv_kernel<L1, L2, LO, SYM, C, EG, true, false, false>,
+                                            tp_bwd_conv_kernel<L1, L2, LO, SYM, C, EG, true, true, true>,
+                                            tp_bwd_conv_kernel<L1, L2, LO, SYM, C, EG, false, true, true>,
+                                            tp_bwd_conv_kernel<L1, L2, LO, SYM, C, EG, false, true, false>};
+    const int k = !g.grad_w ? 0 : g.grad_in1 ? 1 : g.grad_in2 ? 2 : 3;
+    if constexpr (C == 128 && EG > 1) {
+      static const struct PerCu {
+        int n[4];
+        PerCu() {
+          for (int i = 0; i < 4; ++i) n[i] = workgroups_per_cu(reinterpret_cast<const void*>(kernels[i]), C * EG, 0);
+        }
+      } per_cu;
+      if (!wide_round(per_cu.n[k], g.n_rows, g.n_edges, 16)) return false;
+    }
+    hipLaunchKernelGGL(kernels[k], grid, dim3(C * EG), 0, stream, g);
     return true;
   }
 }
@@ -1061,17 +1091,26 @@ bool launch_bwd_send(const TPArgs& g, dim3 grid, hipStream_t stream) {
 // launch_tp's answer when a sender-order backward was asked for a configuration it does not cover
 constexpr int kSendNotApplicable = -100;
 
+// Convolution forward with EG edge groups; false (nothing launched) where 128 channels do without them (32 edges
+// a receiver for a second round: with 512 receivers the time of one group over that of four is then 1.01 to 1.18,
+// with 24 edges 0.95 to 1.08, with 16 0.88 to 0.97).
 template <int L1, int L2, int LO, bool SYM, int EG>
-void launch_fwd_groups(const TPArgs& g, dim3 grid, hipStream_t stream) {
+bool launch_fwd_groups(const TPArgs& g, dim3 grid, hipStream_t stream) {
   using CF = TPConfig<L1, L2, LO, SYM>;
   if (g.C == 128) {
-    if constexpr (EG == 4 && wide_groups<L1, L2, LO, SYM>())
-      hipLaunchKernelGGL((tp_fwd_kernel<L1, L2, LO, SYM, true, true, EG, 128>), grid, dim3(g.C * EG),
-                         sizeof(float) * (size_t)CF::NOUT * g.C, stream, g);
-    return;
+    if constexpr (EG == 4 && wide_groups<L1, L2, LO, SYM>()) {
+      const auto kernel = tp_fwd_kernel<L1, L2, LO, SYM, true, true, EG, 128>;
+      constexpr size_t lds = sizeof(float) * (size_t)CF::NOUT * 128;
+      static const int per_cu = workgroups_per_cu(reinterpret_cast<const void*>(kernel), 128 * EG, lds);
+      if (!wide_round(per_cu, g.n_rows, g.n_edges, 32)) return false;
+      hipLaunchKernelGGL(kernel, grid, dim3(128 * EG), lds, stream, g);
+      return true;
+    }
+    return false;
   }
   const size_t lds = sizeof(float) * (size_t)(EG - 1) * CF::NOUT * g.C;
   hipLaunchKernelGGL((tp_fwd_kernel<L1, L2, LO, SYM, true, true, EG>), grid, dim3(g.C * EG), lds, stream, g);
+  return true;
 }
 
 // Host-side launcher for one configuration.
@@ -1156,10 +1195,10 @@ int launch_tp(const TPArgs& g, bool conv, bool bwd, hipStream_t stream) {
     // 51 with four), as many as the backward with 32
     const int eg = g.C == 64 ? (eg0 + 1) / 2 : eg0;
     if (conv) {
-      if (bc2 && eg >= 4) launch_fwd_groups<L1, L2, LO, SYM, 4>(g, grid, stream);
-      else if (bc2 && eg >= 2) launch_fwd_groups<L1, L2, LO, SYM, 2>(g, grid, stream);
-      else if (bc2) hipLaunchKernelGGL((tp_fwd_kernel<L1, L2, LO, SYM, true, true>), grid, block, 0, stream, g);
-      else hipLaunchKernelGGL((tp_fwd_kernel<L1, L2, LO, SYM, true, false>), grid, block, 0, stream, g);
+      const bool grouped = bc2 && ((eg >= 4 && launch_fwd_groups<L1, L2, LO, SYM, 4>(g, grid, stream)) ||
+                                   (eg >= 2 && launch_fwd_groups<L1, L2, LO, SYM, 2>(g, grid, stream)));
+      if (!grouped && bc2) hipLaunchKernelGGL((tp_fwd_kernel<L1, L2, LO, SYM, true, true>), grid, block, 0, stream, g);
+      else if (!grouped) hipLaunchKernelGGL((tp_fwd_kernel<L1, L2, LO, SYM, true, false>), grid, block, 0, stream, g);
     } else {
       hipLaunchKernelGGL((tp_fwd_kernel<L1, L2, LO, SYM, false, false>), grid, block, 0, stream, g);
     }

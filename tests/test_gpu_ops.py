@@ -774,6 +774,37 @@ def test_tp_conv_edge_groups_128(l1, l2, lo, degrees):
         assert_close(a, b, 2e-5, 2e-5 * (float(b.abs().max()) + 1), f"gradient {k}")
 
 
+@pytest.mark.parametrize("l1,l2,lo", [(2, 3, 3), (2, 2, 2), (1, 1, 1)])
+@pytest.mark.parametrize("n,degree", [(256, 8), (257, 8), (257, 16), (512, 31), (512, 32), (513, 32), (767, 8), (769, 8)])
+def test_tp_conv_edge_group_limits_128(l1, l2, lo, n, degree):
+    """Receivers and edges around the limits between one and four edge groups (products of which one, two or more
+    workgroups fit a CU), against the same receivers among so many others that none is shared by groups; float32
+    sums over `degree` edges in another order."""
+    from flashcart_amd import o3
+    C, more = 128, 800
+    few = random_csr_graph(n, [degree], seed=n)
+    both = torch.cat([few, torch.arange(n, n + more).expand(2, -1)], 1)
+    tp = o3.TensorProduct(l1, l2, lo, C, 1)
+    gen = torch.Generator(device=DEV).manual_seed(n + l1)
+
+    def t(*shape):
+        return torch.randn(*shape, device=DEV, generator=gen)
+
+    e = both.shape[1]
+    big = [t(n + more, (l1 + 1) ** 2 * C), t(e, (l2 + 1) ** 2), t(e, tp.n_total_paths * C)]
+    rows = (n, few.shape[1], few.shape[1])
+    go = None
+    results = []
+    for edges, leaves in ((both, big), (few, [a[:k] for a, k in zip(big, rows)])):
+        leaves = [a.clone().requires_grad_(True) for a in leaves]
+        out = tp(*leaves, edges[0].to(DEV), edges[1].to(DEV))
+        go = t(*out.shape) if go is None else go
+        grads = torch.autograd.grad(out, leaves, go[:out.shape[0]])
+        results.append([out] + list(grads))
+    for k, (want, got) in enumerate(zip(*results)):
+        _close(got, want[:got.shape[0]], f"result {k}")
+
+
 @pytest.mark.parametrize("n", [1, 7, 33, 257, 5003])
 @pytest.mark.parametrize("k,m,act", [(3, 4, 0), (130, 65, 1), (64, 128, 0), (200, 64, 1)])
 def test_wgrad_tiles(n, k, m, act):
