@@ -36,6 +36,11 @@ namespace fc {
 
 constexpr int kNLMaxPerAtom = 1024;  // pairs per receiver held in LDS by the fill kernel
 constexpr int kNLShiftBias = 512;    // shift components packed in 10 bits each: |S| < 512
+// A cell far thinner than the cutoff is left to the host list before anything is launched: beyond 2^20 bins
+// to one side, or 2^18 runs of candidates (nl_visit) for a receiver. Lists of at most 1,024 pairs an atom and 511 images
+// an axis need some 10,000 runs (1,023 x 9 for one thin axis, 4 x 1,024 / pi x 3 for two), more in skewed cells only. A
+// wave takes 1 s for the 3 million runs of a cell of 8 x 0.008 x 0.008 under a cutoff of 4, each with an atom in it.
+constexpr double kNLMaxBinsAway = 1 << 20, kNLMaxRuns = 1 << 18;
 
 struct NLPlan {
   double cell[9], inv[9];
@@ -466,28 +471,26 @@ static int64_t nl_build(int64_t n, const double* pos, const double* cell, const 
   // two atoms closer than the cutoff two bins apart). Periodic axes: D = ceil(reach / width)
   // neighbouring bins each way (several images when the cell is thinner than the cutoff).
   for (int k = 0; k < 3; ++k) {
-    const double span = hi[k] - lo[k];
-    int nbk = (int)std::floor(span / (reach[k] * (1.0 + 1e-6)));
-    nbk = nbk < 1 ? 1 : (nbk > 512 ? 512 : nbk);
-    p.nb[k] = nbk;
+    const double span = hi[k] - lo[k], fit = std::floor(span / (reach[k] * (1.0 + 1e-6)));
+    p.nb[k] = !(fit > 1) ? 1 : (fit > 512 ? 512 : (int)fit);
     p.base[k] = lo[k];
-    p.width[k] = span > 0 ? span / nbk : 1.0;
-    p.D[k] = p.pbc[k] ? (int)std::ceil(reach[k] / p.width[k]) : 1;
   }
   while ((int64_t)p.nb[0] * p.nb[1] * p.nb[2] > nl_max_bins(n)) {  // coarser bins for sparse systems
     int k = 0;
     for (int q = 1; q < 3; ++q)
       if (p.nb[q] > p.nb[k]) k = q;
     p.nb[k] = (p.nb[k] + 1) / 2;
-    p.width[k] = (hi[k] - lo[k]) > 0 ? (hi[k] - lo[k]) / p.nb[k] : 1.0;
-    p.D[k] = p.pbc[k] ? (int)std::ceil(reach[k] / p.width[k]) : 1;
+  }
+  for (int k = 0; k < 3; ++k) {
+    const double span = hi[k] - lo[k];
+    p.width[k] = span > 0 ? span / p.nb[k] : 1.0;
+    const double away = p.pbc[k] ? std::ceil(reach[k] / p.width[k]) : 1.0;
+    if (!(away <= kNLMaxBinsAway)) return -FC_ERR_SHAPE;  // (before it is an integer)
+    p.D[k] = (int)away;
   }
   const int64_t nbins = (int64_t)p.nb[0] * p.nb[1] * p.nb[2];
   p.ns2 = p.pbc[2] ? (2 * p.D[2] + p.nb[2] - 1) / p.nb[2] + 1 : 1;
-  // A cell a million times thinner than the cutoff, or columns of bins beyond 31 bits: the host list's.
-  for (int k = 0; k < 3; ++k)
-    if (p.D[k] < 0 || p.D[k] > (1 << 20)) return -FC_ERR_SHAPE;
-  if ((2.0 * p.D[0] + 1.0) * (2.0 * p.D[1] + 1.0) * p.ns2 > 2147483647.0) return -FC_ERR_SHAPE;
+  if ((2.0 * p.D[0] + 1.0) * (2.0 * p.D[1] + 1.0) * p.ns2 > kNLMaxRuns) return -FC_ERR_SHAPE;
   int32_t* const status = ws.status->status;
   hipLaunchKernelGGL(nl_init_kernel, dim3((unsigned)((nbins + bs - 1) / bs)), dim3(bs), 0, s, nbins, ws.hist, status);
   hipLaunchKernelGGL(nl_bin_kernel, dim3(g_atoms), dim3(bs), 0, s, p, pos, ws.bin, ws.hist);

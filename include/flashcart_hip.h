@@ -466,7 +466,9 @@ int64_t fc_neighbor_list(int64_t n, const double* pos, const double* cell, const
  * memory of fc_neighbor_list_device_workspace(n) bytes. Synchronises `stream` (the pair
  * count is read back). Returns the pair count (outputs written only when it fits in
  * `capacity`), or -fc_status: FC_ERR_BAD_DESC (singular cell, bad cutoff),
- * FC_ERR_SHAPE (more than 1024 pairs for one atom, or a shift component >= 512). */
+ * FC_ERR_SHAPE (more than 1024 pairs for one atom, a shift component >= 512, or, before
+ * anything is launched, a cell thinner than the cutoff by so much that a receiver has more
+ * than 2^18 runs of candidate bins or bins more than 2^20 away). */
 int64_t fc_neighbor_list_device_workspace(int64_t n);
 int64_t fc_neighbor_list_device(int64_t n, const double* pos, const double* cell, const int32_t* pbc,
                                 double cutoff, int64_t capacity, int64_t* out_i, int64_t* out_j,

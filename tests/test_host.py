@@ -474,3 +474,29 @@ def test_operator_kernel_overrides(by_name):
         assert torch.equal(own(x.detach()), 2 * x)
         lib.impl(f"{name}_{key}", lambda x: 7 * x, key)
         assert own(x.detach()) == "registry"
+
+
+@pytest.mark.skipif(torch.cuda.is_available(), reason="the positions here are no device memory")
+@pytest.mark.parametrize("cell,pbc,refused", [
+    (np.diag([8.0, 8.0, 8.0]), (1, 1, 1), False),
+    (np.diag([8.0, 0.008, 9.0]), (1, 1, 1), False),          # 500 images each way along an axis
+    (np.diag([9.0, 0.04, 0.04]), (1, 1, 1), False),          # 100 and 100
+    (np.diag([0.032, 0.016, 9.0]), (1, 1, 1), False),        # 251 x 501 x 2 runs of candidates a receiver
+    (np.diag([0.032, 0.015, 9.0]), (1, 1, 1), True),         # 251 x 535 x 2
+    (np.diag([8.0, 0.0008, 0.0008]), (1, 1, 1), True),       # 100 million
+    (np.diag([8.0, 9.0, 1e-7]), (1, 1, 1), True),            # 4e7 bins away
+    (np.diag([8.0, 1e-9, 9.0]), (1, 1, 1), True),            # 4e9: beyond 32 bits
+    (np.diag([8.0, 9.0, 1e-20]), (1, 1, 1), True),           # 4e20: beyond 64
+    (np.diag([1e-200, 9.0, 1e-90]), (1, 1, 1), True)])
+def test_device_list_refuses_thin_cells(cell, pbc, refused):
+    """fc_neighbor_list_device refuses, before it launches anything, cells so thin that a receiver's search would
+    run for long or its counts would not fit; other cells get as far as the launch, which fails here."""
+    from flashcart_amd import _lib
+    from flashcart_amd.data.neighbors import host_fallback_needed
+    lib = _lib.load()
+    cell = np.ascontiguousarray(cell)
+    flags = np.asarray(pbc, dtype=np.int32)
+    pos, ws = np.zeros((2, 3)), np.zeros(1 << 16, dtype=np.uint8)
+    n = lib.fc_neighbor_list_device(2, pos.ctypes.data, cell.ctypes.data, flags.ctypes.data, 4.0, 0, None, None, None,
+                                    ws.ctypes.data, ws.size, None)
+    assert n < 0 and host_fallback_needed(n) == refused
