@@ -1141,7 +1141,10 @@ __device__ __forceinline__ void wide_body(const WideA& a, bf16x8 (*Bs)[3 * WIDE_
         hi[j][v] = (hi[j][v] + lo[j][v]) * kSplitUnscale;
         probe = fmaf(hi[j][v], 0.f, probe);
       }
-    if (__any(probe != probe)) {  // again in plain float32
+    float late = scale;
+    if (__any(probe != probe)) {
+      // Again in plain float32, with the weights scaled first: x W may overflow where scale x W does not.
+      late = 1.f;
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
         const float* p = w + (int64_t)min(c0 + 32 * j + rl, m - 1) * WIDE_K + 8 * h;
@@ -1150,7 +1153,8 @@ __device__ __forceinline__ void wide_body(const WideA& a, bf16x8 (*Bs)[3 * WIDE_
         for (int q = 0; q < 8; ++q) {
           const f32x4 bv = *reinterpret_cast<const f32x4*>(p + 16 * (q >> 1) + 4 * (q & 1));
 #pragma unroll
-          for (int i = 0; i < 4; ++i) hi[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a.x[q][i], bv[i], hi[j], 0, 0, 0);
+          for (int i = 0; i < 4; ++i)
+            hi[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a.x[q][i], bv[i] * scale, hi[j], 0, 0, 0);
         }
       }
     }
@@ -1160,7 +1164,7 @@ __device__ __forceinline__ void wide_body(const WideA& a, bf16x8 (*Bs)[3 * WIDE_
       for (int v = 0; v < 16; ++v)
 #pragma unroll
         for (int j = 0; j < 2; ++j)
-          __builtin_nontemporal_store(hi[j][v] * scale,
+          __builtin_nontemporal_store(hi[j][v] * late,
                                       reinterpret_cast<gfloat*>(reinterpret_cast<gchar*>(base) + voff[v]) + j * 32);
     } else {
 #pragma unroll
@@ -1168,7 +1172,7 @@ __device__ __forceinline__ void wide_body(const WideA& a, bf16x8 (*Bs)[3 * WIDE_
 #pragma unroll
         for (int j = 0; j < 2; ++j)
           if (row0 + 8 * (v >> 2) + (v & 3) < n && c0 + j * 32 + rl < m)
-            *(reinterpret_cast<gfloat*>(reinterpret_cast<gchar*>(base) + voff[v]) + j * 32) = hi[j][v] * scale;
+            *(reinterpret_cast<gfloat*>(reinterpret_cast<gchar*>(base) + voff[v]) + j * 32) = hi[j][v] * late;
     }
     __syncthreads();
     buf ^= 1;

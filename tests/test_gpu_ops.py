@@ -729,6 +729,32 @@ def test_dense_tiles(n, k, m, act):
     assert bool(((gx.double() - want_gx).abs() <= gx_bound)[rows].all())
 
 
+@pytest.mark.parametrize("n,m", [(1, 256), (129, 320), (128, 330)])
+def test_wide_output_scaled_range(n, m):
+    """The wide output layers where x W leaves float32's range and scale * x W does not (the weights are scaled
+    before they are multiplied), against float64: dense layer and radial MLP. 1e38 is far enough from the limit that
+    no partial sum of the scaled products overflows. The hidden layers' error, exp's included, is below 2^-18."""
+    ops = _ops()
+    g = torch.Generator(device=DEV).manual_seed(n)
+    x, w = torch.randn(n, 64, device=DEV, generator=g) * 1e19, torch.randn(m, 64, device=DEV, generator=g) * 3e19
+    scale = 2.0 ** -9 * 1.25
+    with torch.no_grad():
+        out, _ = ops.dense_fwd(x, w, None, scale, 0)
+    want = scale * (x.double() @ w.double().t())
+    assert float((want / scale).abs().max()) > 3.5e38 and float(want.abs().max()) < 1e38
+    assert bool(((out.double() - want).abs() <= scale * _map_bound(x.double(), w.double(), 64)).all())
+
+    x8, w0, w1 = (torch.randn(*s, device=DEV, generator=g) for s in ((n, 8), (64, 8), (64, 64)))
+    w2 = torch.randn(m, 64, device=DEV, generator=g).clamp(-2.5, 2.5) * 1e38
+    with torch.no_grad():
+        out = ops.radial_mlp_fwd(x8, w0, 0.35, w1, 0.125, w2, scale)
+    h2 = O.silu(0.125 * O.silu(0.35 * x8.double() @ w0.double().t()) @ w1.double().t())
+    want = scale * (h2 @ w2.double().t())
+    assert float((want / scale).abs().max()) > 3.5e38 and float(want.abs().max()) < 1e38
+    bound = scale * (_map_bound(h2, w2.double(), 64) + 2.0 ** -18 * (h2.abs().amax() * w2.double().abs().sum(1)))
+    assert bool(((out.double() - want).abs() <= bound).all())
+
+
 @pytest.mark.parametrize("pairs", [1, 37, 6001])
 def test_dense_bwd_pairs_sizes(pairs):
     """The pair-summed input gradient with few pairs and with enough for its tiled kernel."""
