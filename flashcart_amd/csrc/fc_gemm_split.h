@@ -7,11 +7,13 @@
 // another, added at the end. What is left out is below 2^-24 of a product. Measured against
 // float64 with normal operands, relative 2-norm error at K = 128 / 896 / 8,192: 0.66 / 1.7 / 5.7e-7,
 // against 2.0 / 5.4 / 17e-7 for v_mfma_f32_16x16x4f32, whose chain rounds after every product.
-// Range: bf16 has float32's exponents but its matrix instructions flush subnormal inputs, which the
-// low parts of operands below 2^-109 are; operands are therefore scaled by 2^20 as they are split
-// (and results by 2^-40), which keeps all 24 bits of every normal float32. Results that come out
-// infinite or NaN (an infinite or NaN operand, an operand above 2^107, an overflowing sum) are
-// formed again on the float32 matrix cores, so those follow the IEEE rules as before.
+// Range: the parts of an operand are multiples of its last bit, at least 2^-149, but bf16's smallest
+// subnormal is 2^-133; operands are therefore scaled by 2^20 as they are split (and results by 2^-40),
+// which keeps all bits of every float32, subnormal ones included: the matrix instructions take subnormal
+// parts as they are (relative error 5e-8 at K = 64 from operands of 2^-110 down to 2^-132, less below,
+// where operands have fewer bits). Results that come out infinite or NaN (an infinite or NaN operand, an
+// operand above 2^107, a sum above 2^88) are formed again on the float32 matrix cores, so those follow
+// the IEEE rules as before.
 //
 // Rate: six bf16 MFMAs take 3/8 of the time of the float32 MFMAs they replace, plus 6.5 VALU
 // instructions for each operand element that is split.

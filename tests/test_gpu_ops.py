@@ -670,6 +670,39 @@ def test_linear_special_values(n, fout):
     assert bool((out[41] == 0).all())
 
 
+def test_split_operands_bottom_of_range():
+    """Operands in the last normal binades and subnormal ones keep all their bits in the kernels that split them: map,
+    input gradient (of 64 and 128 columns), weight gradient and wide output, with the small operand on either side,
+    against float64. The results are normal numbers."""
+    ops = _ops()
+    n = 40001
+    g = torch.Generator(device=DEV).manual_seed(5)
+
+    def small(rows, cols):  # rows of 2^-120 to 2^-146
+        e = torch.arange(rows, device=DEV) % 27 + 120
+        return (torch.randn(rows, cols, device=DEV, generator=g).double() * torch.exp2(-e.double())[:, None]).float()
+
+    def large(rows, cols):
+        return torch.randn(rows, cols, device=DEV, generator=g) * 2.0 ** 60
+
+    def check(got, a, b, k, what):
+        a, b = a.double(), b.double()
+        assert bool(((got.double() - a @ b.t()).abs() <= _map_bound(a, b, k)).all()), what
+
+    for left, right in ((small, large), (large, small)):
+        for k, m in ((64, 64), (96, 160)):
+            x, w, go = left(n, k), right(m, k), left(n, m)
+            with torch.no_grad():
+                check(ops.linear_fwd(x, [w], 0, 0, k, m, [1], [1.0], 1.0), x, w, k, (left.__name__, "map", k, m))
+                check(ops.linear_bwd(go, [w], 0, 0, k, m, [1], [1.0], 1.0), go, w.t(), m, (left.__name__, "gradient", k, m))
+        a, b = left(n, 64), right(n, 160)
+        with torch.no_grad():
+            check(ops.dense_wgrad(a, None, 0, b, 1.0, True, False)[0], a.t(), b.t(), n, (left.__name__, "weights"))
+        x, w = left(130, 64), right(320, 64)
+        with torch.no_grad():
+            check(ops.dense_fwd(x, w, None, 1.0, 0)[0], x, w, 64, (left.__name__, "wide"))
+
+
 @pytest.mark.parametrize("n", [1, 15, 33, 64, 65, 1025])
 def test_tp_rows_shared_weight_gradient(n):
     """The gradient of weights shared by all rows: the column sum over the rows in one pass and in parts,
