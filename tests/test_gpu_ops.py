@@ -603,7 +603,9 @@ def _map_bound(x, w, k):
     (50001, 0, 0, 32, 4, [1]), (6001, 1, 1, 32, 33, [1, 2]), (2203, 2, 1, 64, 63, [1, 1, 2]),
     (8129, 0, 0, 96, 65, [1]), (2033, 3, 3, 32, 100, [5, 1, 2, 3]), (1128, 1, 2, 160, 128, [1, 1]),
     # enough tiles for 128-column tiles: two column tiles, the second and the last row tile partial
-    (40001, 0, 0, 32, 200, [1]), (8201, 3, 3, 32, 132, [1, 2, 1, 1])])
+    (40001, 0, 0, 32, 200, [1]), (8201, 3, 3, 32, 132, [1, 2, 1, 1]),
+    # the same in the input gradient (K = 96, 64): columns in two tiles, and in one that is partial
+    (40001, 0, 0, 140, 96, [1]), (8201, 3, 3, 36, 64, [1, 2, 1, 3])])
 def test_linear_tiles(n, lin, lout, fin, fout, paths):
     """The linear maps' kernels at the edges of their tiles (rows, columns, K steps), forward with a residual and
     input gradient, against float64 with an element-wise bound."""
@@ -668,6 +670,41 @@ def test_linear_special_values(n, fout):
         err = (got[rows].double() - want[rows]).abs()
         assert bool((err <= bound)[finite[rows]].all())
     assert bool((out[41] == 0).all())
+
+
+@pytest.mark.parametrize("n,k,fout", [
+    (20000, 64, 64), (20011, 72, 96),     # 64-column tiles, the second with a partial one
+    (40000, 136, 160), (40065, 200, 32)])  # 128-column tiles
+def test_linear_gradient_special_values(n, k, fout):
+    """Infinities, NaN and operands at both ends of float32's range in the gradient that the map's input gradient
+    contracts (rows of tiles, the last one too): IEEE sums, full precision elsewhere, also in the tiles that hold them."""
+    ops = _ops()
+    g = torch.Generator(device=DEV).manual_seed(k)
+    go = torch.randn(n, fout, device=DEV, generator=g)
+    w = torch.randn(fout, k, device=DEV, generator=g)
+    w[7, 5] = 0.0
+    w[9, k - 1] = float("inf")
+    w[0, k - 1] = 0.0  # (3.4e38 below times a weight above 1 is infinite in float32 alone)
+    w[11] *= 1e-30
+    go[1, 7] = float("inf")
+    go[33, 9] = float("nan")
+    go[n - 1, 3] = float("-inf")
+    go[n - 2, 9] = 0.0  # 0 x inf
+    go[40] *= 1e-36
+    go[41] = 0.0
+    go[42] *= 1e30
+    go[43, 0] = 3.4e38  # rounds to infinity in 16 bits
+    with torch.no_grad():
+        got = ops.linear_bwd(go, [w], 0, 0, k, fout, [1], [1e-3], 1.0)
+    unscaled = go.double() @ w.double()
+    assert torch.equal(got.isnan(), unscaled.isnan())
+    assert torch.equal(got[unscaled.isinf()], unscaled[unscaled.isinf()].float())
+    rows, cols = torch.isfinite(go).all(1), torch.isfinite(w).all(0)
+    a, b = go[rows].double(), w[:, cols].double()
+    err = (got[rows][:, cols].double() - 1e-3 * (a @ b)).abs()
+    fits = (a.abs() @ b.abs()) < 3e38  # no partial sum overflows
+    assert bool((err <= 1e-3 * _map_bound(a, b.t(), fout) + 2.0 ** -126)[fits].all()) and float(fits.double().mean()) > 0.99
+    assert bool((got[41][cols] == 0).all())
 
 
 def test_split_operands_bottom_of_range():
