@@ -1747,7 +1747,11 @@ struct WgradBatch {
 // 2 x 2, each (TO / 2) x (TJ / 2) outputs in 32x32x16 blocks; the next step's rows load during the current
 // step's MFMAs.
 // Weight gradients of the product linear (K = 512 to 896, N = 128; with the reduction), against the float32
-// matrix instructions before it: 25,000 nodes 1,197 -> 858 us, 6,691 nodes 287 -> 227 us.
+// matrix instructions before it: 25,000 nodes 1,197 -> 858 us, 6,691 nodes 287 -> 227 us; 64-wide maps, l <= 2:
+// 25,000 nodes 99 -> 71 us, 6,700 nodes 37 us either way. With 64 x 64 tiles a launch has 0.5 to 1 us more to do before
+// its first rows are there (row cursors and addresses in scalar registers): 8 rows 5.1 -> 5.9 us, 300 rows 18.0 -> 19.0.
+// Steps that do not exist are not loaded (8 rows 6.7 us with one); loads at one place of the loop, for half the
+// code, gained nothing there and cost 3% at 25,000 rows.
 template <int TO, int TJ, bool ACT>
 __global__ void __launch_bounds__(256, 2) wgrad_kernel(WgradBatch wb) {
   constexpr int RK = 32;                    // rows per step
@@ -1879,14 +1883,14 @@ __global__ void __launch_bounds__(256, 2) wgrad_kernel(WgradBatch wb) {
     for (int j = 0; j < FJ; ++j) hi[i][j] = lo[i][j] = floatx16{};
 
   if (r_begin < r_end) {
-    seek(r_begin);
+    if (r_begin + RK <= r_end) seek(r_begin);  // (else load does)
     load(r_begin);
   }
   for (int r0 = r_begin; r0 < r_end; r0 += RK) {
     store(r0);
     __syncthreads();
     __builtin_amdgcn_sched_barrier(0);
-    load(min(r0 + RK, r_end - 1));  // (issued on every path; the last turn's are not used)
+    if (r0 + RK < r_end) load(r0 + RK);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
