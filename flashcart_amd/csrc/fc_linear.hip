@@ -1,4 +1,5 @@
-// Equivariant linear maps and dense layers on the fp32 matrix cores (MFMA).
+// Equivariant linear maps and dense layers of float32 operands on the matrix cores (MFMA): bf16 ones with split
+// operands for most launches, fp32 ones for the others.
 //
 // Per rank l the equivariant map is a GEMM with M = n*(2l+1) rows (one per node and
 // component), K = in_features*in_paths[l], N = out_features, and one weight matrix
@@ -63,7 +64,7 @@ struct GemmBatch {
   int32_t trans_b;    // 1: B(k, o) = W[o*K + k] (forward); 0: B(k, o) = W[k*N + o] (input gradient)
   int32_t act;        // 1: rescaled SiLU epilogue (fwd)
   int32_t act_bwd;    // 1: rescaled SiLU derivative prologue on A (dgrad)
-  int32_t pair_sum;   // 1: A rows hold two K-long halves, multiplied as their sum (pipelined kernel only)
+  int32_t pair_sum;   // 1: A rows hold two K-long halves, multiplied as their sum (one rank, at most 64 columns)
 };
 
 __device__ __forceinline__ float sigmoidf_(float x) { return 1.0f / (1.0f + __expf(-x)); }
@@ -380,7 +381,7 @@ __global__ void __launch_bounds__(256) gemm_kernel(GemmBatch gb) {
 }
 
 // ---------------------------------------------------------------------------------------
-// Pair-sum GEMM: D = scale (A_lo + A_hi) W^T, where every A row is the sum of two halves of K floats,
+// Pair-sum GEMM of at most 64 columns: D = scale (A_lo + A_hi) W^T, where every A row is the sum of two halves of K floats,
 // A[r, 0:K] and A[r, K:2K], or rows a_lo[r] and a_hi[r] of A when the rank gives those index arrays;
 // both halves go to LDS and are added as the MFMA operands are read, so the MFMA work is that of K
 // (the radial output layer's input gradient over edge pairs, whose two edges share the layer's
@@ -429,10 +430,6 @@ __device__ __forceinline__ void pipe_barrier() {
 // s_waitcnt immediate (gfx9 encoding): vector-memory count <= vm, LDS count <= lgkm, no export wait
 #define FC_WAITCNT_IMM(vm, lgkm) (((vm) & 0xF) | ((((vm) >> 4) & 3) << 14) | (0x7 << 4) | (((lgkm) & 0xF) << 8))
 
-struct PipeTile {
-  int ri, r0, c0, K;
-};
-
 constexpr int PAIR_T = 64;  // output tile edge
 
 __global__ void __launch_bounds__(256, 2) gemm_pairsum_kernel(GemmBatch gb) {
@@ -455,62 +452,26 @@ __global__ void __launch_bounds__(256, 2) gemm_pairsum_kernel(GemmBatch gb) {
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   const int wm = wave / WN, wn = wave % WN;
   const int G = gridDim.x, b = blockIdx.x;
-  // Tiles of this workgroup: a contiguous range holding 1/G of the batch's K steps (ranks
-  // differ in K, so equal tile counts would not be equal work). Workgroups of one XCD
-  // (hardware block b runs on XCD b % 8) take neighbouring ranges, so an XCD's L2 serves
-  // one contiguous run of A rows.
+  // This workgroup's row tiles: a contiguous range of 1/G of them. Workgroups of one XCD (hardware
+  // block b runs on XCD b % 8) take neighbouring ranges, so an XCD's L2 serves one contiguous run of
+  // A rows. (Uniform; kept in scalar registers so the tile loop's bookkeeping stays scalar.)
   const int v = (G >= 8 && G % 8 == 0) ? (b % 8) * (G / 8) + b / 8 : b;
-  int64_t work = 0;
-#pragma unroll
-  for (int q = 0; q < FC_MAX_RANKS; ++q)
-    if (q < gb.n_ranks) work += (int64_t)gb.r[q].tiles_m * gb.r[q].tiles_n * (gb.r[q].K / 32);
-  // first tile whose first K step (counted over the whole batch) is at or after step s
-  auto tile_at = [&](int64_t s) -> int {
-    int64_t base = 0;
-#pragma unroll
-    for (int q = 0; q < FC_MAX_RANKS; ++q) {
-      if (q >= gb.n_ranks) break;
-      const GemmRank& g = gb.r[q];
-      const int64_t ks = g.K / 32, n = (int64_t)g.tiles_m * g.tiles_n;
-      if (n > 0 && s <= base + (n - 1) * ks) {
-        const int64_t d = s - base;
-        return g.tile_base + (int)(d <= 0 ? 0 : (d + ks - 1) / ks);
-      }
-      base += n * ks;
-    }
-    return gb.total_tiles;
-  };
-  // (uniform; kept in scalar registers so the tile loop's bookkeeping stays scalar)
-  const int t_first = __builtin_amdgcn_readfirstlane(tile_at(((int64_t)v * work + G - 1) / G));
-  const int t_end = __builtin_amdgcn_readfirstlane(tile_at(((int64_t)(v + 1) * work + G - 1) / G));
-  constexpr int t_step = 1;
-  auto decode = [&](int tile) -> PipeTile {
-    int ri = 0;
-#pragma unroll
-    for (int q = 1; q < FC_MAX_RANKS; ++q)
-      if (q < gb.n_ranks && tile >= gb.r[q].tile_base) ri = q;
-    ri = __builtin_amdgcn_readfirstlane(ri);  // uniform: keeps the rank's fields in scalar loads
-    const GemmRank& g = gb.r[ri];
-    const int local = tile - g.tile_base;
-    if (g.tiles_n == 1) return PipeTile{ri, local * BM, 0, g.K};  // uniform: no division
-    return PipeTile{ri, (local / g.tiles_n) * BM, (local % g.tiles_n) * BN, g.K};
-  };
+  const GemmRank& g = gb.r[0];
+  const int t_first = __builtin_amdgcn_readfirstlane((int)(((int64_t)v * gb.total_tiles + G - 1) / G));
+  const int t_end = __builtin_amdgcn_readfirstlane((int)(((int64_t)(v + 1) * gb.total_tiles + G - 1) / G));
 
   // ---- producer: direct loads of K steps in tile order
   int p_tile = t_first, p_k = 0, n_issued = 0;
-  PipeTile pt{0, 0, 0, 32};
   const float* a_src[A_DMA];
   const float* a_src2[A_DMA];  // second halves
   const float* b_src[B_DMA];
   auto p_setup = [&]() {
     if (p_tile >= t_end) return;
-    pt = decode(p_tile);
-    const GemmRank& g = gb.r[pt.ri];
 #pragma unroll
     for (int j = 0; j < A_DMA; ++j) {
       const int s = (j * 4 + wave) * 64 + lane;
       const int row = s >> 3, c = (s & 7) ^ pipe_swz(row);
-      const int grow = min(pt.r0 + row, g.M - 1);
+      const int grow = min(p_tile * BM + row, g.M - 1);
       if (g.a_lo) {
         // Gathered halves. Using these loads waits for every outstanding vector load, the
         // direct loads of the ring included (once per tile).
@@ -525,7 +486,7 @@ __global__ void __launch_bounds__(256, 2) gemm_pairsum_kernel(GemmBatch gb) {
     for (int j = 0; j < B_DMA; ++j) {
       const int s = (j * 4 + wave) * 64 + lane;
       const int col = s >> 3, c = (s & 7) ^ pipe_swz(col);
-      const int gcol = min(pt.c0 + col, g.N - 1);
+      const int gcol = min(col, g.N - 1);
       b_src[j] = g.B + (int64_t)gcol * g.K + 4 * c;
     }
   };
@@ -542,17 +503,15 @@ __global__ void __launch_bounds__(256, 2) gemm_pairsum_kernel(GemmBatch gb) {
     for (int j = 0; j < B_DMA; ++j) lds_dma16(b_src[j] + p_k, bs + 4096u * j + wave_lds);
     ++n_issued;
     p_k += 32;
-    if (p_k >= pt.K) {
+    if (p_k >= g.K) {
       p_k = 0;
-      p_tile += t_step;
+      ++p_tile;
       p_setup();
     }
   };
 
   // ---- consumer
   int c_tile = t_first, c_k = 0, n_done = 0;
-  PipeTile ct{0, 0, 0, 32};
-  if (c_tile < t_end) ct = decode(c_tile);
   accv acc[FM][FN];
 #pragma unroll
   for (int i = 0; i < FM; ++i)
@@ -597,20 +556,19 @@ __global__ void __launch_bounds__(256, 2) gemm_pairsum_kernel(GemmBatch gb) {
   };
 
   auto epilogue = [&]() {
-    const GemmRank& g = gb.r[ct.ri];
-    const int M = g.M, N = g.N;
+    const int M = g.M, N = g.N, r0 = c_tile * BM;
     const float scale = g.scale;
     // Rows are addressed from the tile's first row (a uniform base) with 32-bit byte offsets (the
     // caller bounds them), columns j > 0 as immediate offsets.
-    gfloat* const Dt = uniform_gptr(g.D + (int64_t)ct.r0 * g.d_row);
-    const int col0 = ct.c0 + wn * TN + (lane & (MI - 1));  // this lane's column in block j = 0
-    const bool all_cols = ct.c0 + BN <= N;                  // uniform
+    gfloat* const Dt = uniform_gptr(g.D + (int64_t)r0 * g.d_row);
+    const int col0 = wn * TN + (lane & (MI - 1));  // this lane's column in block j = 0
+    const bool all_cols = BN <= N;                          // uniform
 #pragma unroll
     for (int i = 0; i < FM; ++i)
 #pragma unroll
       for (int v = 0; v < NV; ++v) {
         const int row = wm * TM + i * MI + 4 * (lane >> 4) + v;  // block row of value v
-        if (ct.r0 + row >= M) continue;
+        if (r0 + row >= M) continue;
         const uint32_t off = 4u * (uint32_t)(row * (int)g.d_row + col0);
         gfloat* const d = reinterpret_cast<gfloat*>(reinterpret_cast<gchar*>(Dt) + off);
 #pragma unroll
@@ -632,12 +590,11 @@ __global__ void __launch_bounds__(256, 2) gemm_pairsum_kernel(GemmBatch gb) {
     else compute(as, bs, std::false_type{});
     ++n_done;
     c_k += 32;
-    if (c_k >= ct.K) {
+    if (c_k >= g.K) {
       epilogue();
       c_k = 0;
-      c_tile += t_step;
+      ++c_tile;
       more = c_tile < t_end;
-      if (more) ct = decode(c_tile);
     }
   };
 
@@ -668,16 +625,11 @@ static bool split_ok(const GemmBatch& gb, int n_ranks) {
 }
 
 static int launch_pairsum(GemmBatch gb, hipStream_t s) {
-  GemmRank& g = gb.r[0];
+  const GemmRank& g = gb.r[0];
   if (g.K < 32 || (g.K & 31) || (g.a_row & 3) || ((uintptr_t)g.A & 15) || ((uintptr_t)g.B & 15)) return FC_ERR_SHAPE;
-  if (64 * g.d_row + g.N >= (int64_t(1) << 29)) return FC_ERR_SHAPE;  // the epilogue's byte offsets
-  g.tiles_m = (g.M + PAIR_T - 1) / PAIR_T;
-  g.tiles_n = (g.N + PAIR_T - 1) / PAIR_T;
-  g.tile_base = 0;
-  const int64_t total = (int64_t)g.tiles_m * g.tiles_n;
+  if (g.N > PAIR_T || 64 * g.d_row + g.N >= (int64_t(1) << 29)) return FC_ERR_SHAPE;  // one column tile; byte offsets
+  const int64_t total = (g.M + (int64_t)PAIR_T - 1) / PAIR_T;
   if (total == 0) return FC_OK;
-  if (total > 0x7fffffff) return FC_ERR_SHAPE;
-  gb.n_ranks = 1;
   gb.total_tiles = (int32_t)total;
   int64_t grid = 2 * (int64_t)device_cu_count();
   if (grid > total) grid = total;
