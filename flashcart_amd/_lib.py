@@ -214,8 +214,13 @@ def require_device(name: str, t: torch.Tensor, dtype: torch.dtype = torch.float3
 
 
 def contig(name: str, t: torch.Tensor, dtype: torch.dtype = torch.float32) -> torch.Tensor:
-    require_device(name, t, dtype)
-    t = t.resolve_neg()  # (a negated view's memory holds the values before negation)
+    """``t``, checked, such that its memory holds its values in order: contiguous, and neither a negated view (whose
+    memory holds the values before negation) nor a zero tensor (which has none). Runs several times per
+    operator call, so plain tensors take one function call here."""
+    if not t.is_cuda or t.dtype != dtype:
+        require_device(name, t, dtype)
+    if t.is_neg() or t._is_zerotensor():
+        return t.clone(memory_format=torch.contiguous_format)
     return t if t.is_contiguous() else t.contiguous()
 
 

@@ -107,7 +107,7 @@ def _i32(name: str, t: Optional[Tensor]) -> Optional[Tensor]:
         raise RuntimeError(f"`{name}` must be on a ROCm device, got {t.device}.")
     if t.dtype != torch.int32:
         t = t.to(torch.int32)
-    return t.contiguous()
+    return _lib.contig(name, t, torch.int32)
 
 
 @functools.lru_cache(maxsize=256)
@@ -180,12 +180,16 @@ _EXACT_ITEM = {"List[int]": int, "List[float]": float}
 _IMPLS = getattr(torch.library, "_impls", frozenset())
 
 
+_CAN_TELL = None not in _QUERIES
+_modes, _functions, _functorch, _tracing, _profiler = _QUERIES
+_is_compiling, _forward_ad = torch.compiler.is_compiling, torch.autograd.forward_ad
+
+
 def _observed() -> bool:
-    if torch.compiler.is_compiling() or None in _QUERIES:
-        return True
-    modes, functions, functorch, tracing, profiler = _QUERIES
-    return bool(modes() or functions() or functorch() is not None or tracing() is not None or profiler()
-                or getattr(torch.autograd.forward_ad, "_current_level", 0) >= 0)
+    """(A default device, set by torch.set_default_device or with torch.device(...), is a function mode too: under
+    one every call goes through the registered operators and pays for their argument handling.)"""
+    return (_is_compiling() or not _CAN_TELL or _modes() > 0 or _functions() > 0 or _functorch() is not None
+            or _tracing() is not None or _profiler() or getattr(_forward_ad, "_current_level", 0) >= 0)
 
 
 class Operator(torch.library.CustomOpDef):
@@ -193,10 +197,11 @@ class Operator(torch.library.CustomOpDef):
     ``autograd.Function`` of the same formula where a gradient is wanted, without the operator registry's
     argument handling, which costs more host time (100 us for the 24 arguments of ``tp_fwd``) than the kernels
     of a small call take. Anything that has to see or rewrite the operator itself (``_observed``, tensor
-    subclasses, tensors that are not on a GPU or whose memory does not hold their values, as a negated view's)
-    and every call that the registry would convert or refuse (keywords, arguments of other types or counts)
-    goes through the registered operator ``op``; both run the same implementation and the same backward. Once
-    somebody registers a kernel or an autocast rule of their own for it, every call goes there."""
+    subclasses, tensors that are not on a GPU) and every call that the registry would convert or refuse
+    (keywords, arguments of other types or counts) goes through the registered operator ``op``; both run the
+    same implementation and the same backward. (The registry also writes out negated views and zero tensors;
+    here ``_lib.contig`` and ``_i32`` do, where an implementation takes a tensor's address.) Once somebody
+    registers a kernel or an autocast rule of their own for it, every call goes there."""
 
     overridden = False
 
@@ -250,10 +255,7 @@ class Operator(torch.library.CustomOpDef):
         if not self.required <= len(args) <= len(self.exact):
             return False
         for a, exact in zip(args, self.exact):
-            if type(a) not in exact:
-                return False
-            # (the dispatcher writes out negated views and zero tensors before it calls the implementation)
-            if isinstance(a, Tensor) and (not a.is_cuda or a.is_neg() or a._is_zerotensor()):
+            if type(a) not in exact or (exact[0] is Tensor and a is not None and not a.is_cuda):
                 return False
         return all(type(x) is item for k, item in self.items if k < len(args) for x in args[k])
 
