@@ -1003,8 +1003,10 @@ __device__ __forceinline__ void wide_load_a(const float* row, int h, WideA& a) {
 // Bs holds two weight chunks: block (column block j, k chunk c) of 64 16-byte entries per part, entry
 // (column % 32 ^ 2 (2 c + h)) + 32 h holding k = 16 c + 8 h .. + 7. Every thread of the workgroup calls it.
 // FULL: every row and column of the block is in range, so the stores are unconditional and the
-// compiler can count them as outstanding where it waits for the next weight chunk.
-template <bool FULL>
+// compiler can count them as outstanding where it waits for the next weight chunk. LONG: rows of
+// kWideLong elements or more, whose offsets are formed in 64 bits as they are needed.
+constexpr int kWideLong = 1 << 22;  // (from here on a block's byte offsets, 128 m 4, leave 31 bits)
+template <bool FULL, bool LONG = false>
 __device__ __forceinline__ void wide_body(const WideA& a, bf16x8 (*Bs)[3 * WIDE_PART], int64_t n, int m,
                                           const float* __restrict__ w, float scale, float* __restrict__ out,
                                           int64_t r0) {
@@ -1038,12 +1040,14 @@ __device__ __forceinline__ void wide_body(const WideA& a, bf16x8 (*Bs)[3 * WIDE_
       Bs[buf][2 * WIDE_PART + e] = s.l;
     }
   };
-  // element offset of this lane's 16 output rows from the block's first element (the caller keeps
-  // 128 m 4 below 2^31), so a store is a wave-uniform base plus a 32-bit offset
+  // offset of this lane's 16 output rows from the block's first element, so that a store is a wave-uniform
+  // base plus a 32-bit offset
   uint32_t voff[16];  // bytes
+  if constexpr (!LONG) {
 #pragma unroll
-  for (int v = 0; v < 16; ++v)
-    voff[v] = (uint32_t)((wave * 32 + 4 * h + 8 * (v >> 2) + (v & 3)) * m + rl) * 4u;
+    for (int v = 0; v < 16; ++v)
+      voff[v] = (uint32_t)((wave * 32 + 4 * h + 8 * (v >> 2) + (v & 3)) * m + rl) * 4u;
+  }
   gfloat* const blk = uniform_gptr(out + r0 * m);
   const int64_t row0 = r0 + wave * 32 + 4 * h;
 
@@ -1123,17 +1127,22 @@ __device__ __forceinline__ void wide_body(const WideA& a, bf16x8 (*Bs)[3 * WIDE_
       for (int v = 0; v < 16; ++v)
 #pragma unroll
         for (int j = 0; j < 2; ++j)
-          if (row0 + 8 * (v >> 2) + (v & 3) < n && c0 + j * 32 + rl < m)
-            *(reinterpret_cast<gfloat*>(reinterpret_cast<gchar*>(base) + voff[v]) + j * 32) = hi[j][v] * late;
+          if (row0 + 8 * (v >> 2) + (v & 3) < n && c0 + j * 32 + rl < m) {
+            gfloat* const p = LONG ? base + (int64_t)(wave * 32 + 4 * h + 8 * (v >> 2) + (v & 3)) * m + rl
+                                   : reinterpret_cast<gfloat*>(reinterpret_cast<gchar*>(base) + voff[v]);
+            p[j * 32] = hi[j][v] * late;
+          }
     }
     __syncthreads();
     buf ^= 1;
   }
 }
 
+template <bool LONG>  // (a kernel of its own: the body is long, and code that is not run costs small calls time too)
 __device__ __forceinline__ void wide_out(const WideA& a, bf16x8 (*Bs)[3 * WIDE_PART], int64_t n, int m,
                                          const float* __restrict__ w, float scale, float* __restrict__ out, int64_t r0) {
-  if (r0 + WIDE_BM <= n && m % WIDE_BN == 0) wide_body<true>(a, Bs, n, m, w, scale, out, r0);
+  if constexpr (LONG) wide_body<false, true>(a, Bs, n, m, w, scale, out, r0);
+  else if (r0 + WIDE_BM <= n && m % WIDE_BN == 0) wide_body<true>(a, Bs, n, m, w, scale, out, r0);
   else wide_body<false>(a, Bs, n, m, w, scale, out, r0);
 }
 
@@ -1145,6 +1154,7 @@ static dim3 wide_grid(int64_t blocks, int m) {
   return dim3((unsigned)blocks, (unsigned)parts);
 }
 
+template <bool LONG>
 __global__ void __launch_bounds__(256, 2) gemm_wide_kernel(int64_t n, int m, const float* __restrict__ x,
                                                             const float* __restrict__ w, float scale,
                                                             float* __restrict__ out) {
@@ -1153,7 +1163,7 @@ __global__ void __launch_bounds__(256, 2) gemm_wide_kernel(int64_t n, int m, con
   const int64_t r0 = (int64_t)blockIdx.x * WIDE_BM, row = r0 + 32 * (t >> 6) + (t & 31);
   WideA a;
   wide_load_a(x + (row < n ? row : n - 1) * WIDE_K, (t >> 5) & 1, a);  // rows past n are not stored
-  wide_out(a, Bs, n, m, w, scale, out, r0);
+  wide_out<LONG>(a, Bs, n, m, w, scale, out, r0);
 }
 
 // ---- Radial MLP with two hidden layers of 64 (reference InteractionLayer.radial_mlp,
@@ -1314,7 +1324,7 @@ __device__ __forceinline__ void acc_to_rows(const floatx16 (&acc)[2], float* As,
 
 // HIDDEN: stop after the second hidden layer and write its activation h2 (n x 64) instead of
 // the output layer (the first interaction layer's species density takes h2 itself).
-template <bool HIDDEN>
+template <bool HIDDEN, bool LONG = false>
 __global__ void __launch_bounds__(256, 2) radial_mlp_fwd_kernel(int64_t n, int n_in, const float* __restrict__ x,
                                                                  const float* __restrict__ w0, float s0,
                                                                  const float* __restrict__ w1, float s1, int m,
@@ -1363,7 +1373,7 @@ __global__ void __launch_bounds__(256, 2) radial_mlp_fwd_kernel(int64_t n, int n
   WideA a;
   wide_load_a(As + (wave * 32 + (lane & 31)) * WIDE_P, lane >> 5, a);
   __syncthreads();  // reads of h2 and of both weight matrices done before the weight chunks overwrite them
-  wide_out(a, lds.wide, n, m, w2, s2, out, r0);
+  wide_out<LONG>(a, lds.wide, n, m, w2, s2, out, r0);
 }
 
 // Input gradient of the two hidden layers: given gh2 = dL/dh2 (n, 64),
@@ -1467,12 +1477,10 @@ extern "C" int fc_dense_fwd(int64_t n, int32_t k, int32_t m, const float* x, con
   if (n == 0) return FC_OK;
   if (!x || !w || !out) return FC_ERR_NULL;
   if (n > 0x7fffffff) return FC_ERR_SHAPE;
-  // (output rows are addressed with 32-bit byte offsets in a block: 128 m 4 < 2^31)
-  if (k == WIDE_K && m >= 4 * WIDE_BN && m < (1 << 22) && !bias && act == 0 && ((uintptr_t)x & 15) == 0 &&
-      ((uintptr_t)w & 15) == 0) {
+  if (k == WIDE_K && m >= 4 * WIDE_BN && !bias && act == 0 && ((uintptr_t)x & 15) == 0 && ((uintptr_t)w & 15) == 0) {
     const int64_t blocks = (n + WIDE_BM - 1) / WIDE_BM;
-    hipLaunchKernelGGL(gemm_wide_kernel, wide_grid(blocks, m), dim3(256), 0, (hipStream_t)stream, n, m, x, w, scale,
-                       out);
+    const auto kernel = m < kWideLong ? gemm_wide_kernel<false> : gemm_wide_kernel<true>;
+    hipLaunchKernelGGL(kernel, wide_grid(blocks, m), dim3(256), 0, (hipStream_t)stream, n, m, x, w, scale, out);
     FC_LAUNCH_CHECK();
     return FC_OK;
   }
@@ -1517,9 +1525,9 @@ extern "C" int fc_radial_mlp_fwd(int64_t n, int32_t n_in, const float* x, const 
   if (((uintptr_t)w2 & 15) != 0) return FC_ERR_SHAPE;  // weight chunks load as float4
   const int64_t blocks = (n + WIDE_BM - 1) / WIDE_BM;
   if (blocks > 0x7fffffff) return FC_ERR_SHAPE;
-  if (m >= (1 << 22)) return FC_ERR_SHAPE;  // 32-bit byte offsets inside a block: 128 m 4 < 2^31
-  hipLaunchKernelGGL(radial_mlp_fwd_kernel<false>, wide_grid(blocks, m), dim3(256), 0, (hipStream_t)stream, n,
-                     (int)n_in, x, w0, s0, w1, s1, (int)m, w2, s2, out);
+  const auto kernel = m < kWideLong ? radial_mlp_fwd_kernel<false, false> : radial_mlp_fwd_kernel<false, true>;
+  hipLaunchKernelGGL(kernel, wide_grid(blocks, m), dim3(256), 0, (hipStream_t)stream, n, (int)n_in, x, w0, s0, w1, s1,
+                     (int)m, w2, s2, out);
   FC_LAUNCH_CHECK();
   return FC_OK;
 }

@@ -825,6 +825,28 @@ def test_wide_output_scaled_range(n, m):
     assert bool(((out.double() - want).abs() <= bound).all())
 
 
+@pytest.mark.parametrize("m", [(1 << 22) - 1, 1 << 22, (1 << 23) + 5])
+def test_wide_output_of_millions_of_columns(m):
+    """Rows of a wide output longer than 32-bit byte offsets within a row block reach (128 m 4 from 2^31 on): radial
+    MLP and dense layer, two row blocks of which the second is partial, against float64. The hidden layers' error,
+    exp's included, is below 2^-18."""
+    ops = _ops()
+    n = 130
+    g = torch.Generator(device=DEV).manual_seed(m)
+    x8, w0, w1 = (torch.randn(*s, device=DEV, generator=g) for s in ((n, 8), (64, 8), (64, 64)))
+    w2 = torch.randn(m, 64, device=DEV, generator=g)
+    h2 = O.silu(0.125 * O.silu(0.35 * x8.double() @ w0.double().t()) @ w1.double().t())
+    with torch.no_grad():
+        out = ops.radial_mlp_fwd(x8, w0, 0.35, w1, 0.125, w2, 0.125)
+        dense, _ = ops.dense_fwd(h2.float(), w2, None, 0.125, 0)
+    for c in range(0, m, 1 << 20):
+        w = w2[c:c + (1 << 20)].double()
+        want = 0.125 * (h2 @ w.t())
+        bound = 0.125 * (_map_bound(h2, w, 64) + 2.0 ** -18 * (h2.abs().amax() * w.abs().sum(1)))
+        for got in (out, dense):
+            assert bool(((got[:, c:c + (1 << 20)].double() - want).abs() <= bound).all()), c
+
+
 @pytest.mark.parametrize("pairs", [1, 37, 6001])
 def test_dense_bwd_pairs_sizes(pairs):
     """The pair-summed input gradient with few pairs and with enough for its tiled kernel."""
