@@ -1162,3 +1162,34 @@ def test_tp_conv_some_gradients(C, l1, l2, lo, degrees):
                 _close(a, b, f"gradient {k} of {need}")
             else:
                 assert a.numel() == 0
+
+
+@pytest.mark.parametrize("C", [32, 64, 128])
+@pytest.mark.parametrize("degrees", [(4, 0, 2, 34, 66), (17, 16, 15) * 256])
+def test_tp_conv_some_gradients_paired(C, degrees):
+    """Each subset of the gradients with one weight row for two edges: as with the rows written out per edge (the same
+    kernels, which read the same values), for pairs of arbitrary edges."""
+    ops = _ops()
+    from flashcart_amd.o3._graph import build_graph
+    l1, l2, lo = 2, 3, 3
+    ei = random_csr_graph(len(degrees), degrees, seed=C, allow_self=True)
+    graph = build_graph(ei.to(DEV), len(degrees))
+    g = torch.Generator(device=DEV).manual_seed(C)
+    meta = ops.tp_meta(l1, l2, lo, C, 1, False, False)
+    n, e = len(degrees), ei.shape[1]
+    assert e % 2 == 0
+    slot = torch.randperm(e, device=DEV, generator=g).to(torch.int32)
+    in1, in2, w, go = (torch.randn(*s, device=DEV, generator=g) for s in (
+        (n, (l1 + 1) ** 2 * C), (e, (l2 + 1) ** 2), (e // 2, meta[-1] * C), (n, sum(meta[2]))))
+
+    def run(weights, pairs, *need):
+        return ops.tp_bwd(go, in1, in2, weights, graph.idx_i, graph.idx_j, l1, l2, lo, C, 1, False, False, *meta, False,
+                          *need, graph.rowptr, graph.sender_perm, graph.sender_ptr, 0.7, pairs)
+
+    for mask in range(1, 8):
+        need = [bool(mask & b) for b in (1, 2, 4)]
+        for k, (a, b, on) in enumerate(zip(run(w, slot, *need), run(w[(slot >> 1).long()], None, *need), need)):
+            if on:
+                _close(a, b, f"gradient {k} of {need}")
+            else:
+                assert a.numel() == 0 and b.numel() == 0
