@@ -1146,11 +1146,26 @@ __device__ __forceinline__ void wide_out(const WideA& a, bf16x8 (*Bs)[3 * WIDE_P
   else wide_body<false>(a, Bs, n, m, w, scale, out, r0);
 }
 
-// Row blocks x column parts of the wide kernels: two workgroups per CU where the columns allow it.
-static dim3 wide_grid(int64_t blocks, int m) {
-  const int64_t chunks = (m + WIDE_BN - 1) / WIDE_BN, want = 2 * (int64_t)device_cu_count();
-  int64_t parts = blocks > 0 ? (want + blocks - 1) / blocks : 1;
-  if (parts > chunks) parts = chunks;
+// Row blocks x column parts of the wide kernels. Each part repeats the block's work before its columns, `fixed` column
+// chunks' worth (4 for the radial MLP, whose parts all form the hidden layers, 1 for a dense layer). Two workgroups on
+// a CU take `pair` fifths of one's time (8 and 7), k more 0.8 k times. The number of parts with the least time by that,
+// for up to two row blocks a CU. Radial MLP, microseconds, one part / as many as 512 workgroups have room for / this rule:
+// 235 blocks, 160 columns 23 / 34 / 23, 2,176 columns 89 / 87 / 73; 128 blocks 22 / 24 / 19 and 84 / 51 / 51; 6 blocks
+// 19 / 15 / 15 and 82 / 16 / 16. Dense layer, 235 blocks, 2,176 columns 78 / 74 / 63.
+static dim3 wide_grid(int64_t blocks, int m, int fixed, int pair) {
+  const int64_t chunks = (m + (int64_t)WIDE_BN - 1) / WIDE_BN, cus = device_cu_count();
+  int64_t parts = 1, least = -1;
+  for (int64_t p = 1; p <= chunks && (p == 1 || (blocks <= 2 * cus && blocks * p <= 8 * cus)); ++p) {
+    const int64_t per_cu = (blocks * p + cus - 1) / cus;
+    const int64_t time = (fixed + (chunks + p - 1) / p) * (per_cu <= 1 ? 5 : per_cu == 2 ? pair : 4 * per_cu);
+    if (least < 0 || time < least) {
+      least = time;
+      parts = p;
+    }
+  }
+  return dim3((unsigned)blocks, (unsigned)parts);
+}
+  }
   return dim3((unsigned)blocks, (unsigned)parts);
 }
 
@@ -1480,7 +1495,7 @@ extern "C" int fc_dense_fwd(int64_t n, int32_t k, int32_t m, const float* x, con
   if (k == WIDE_K && m >= 4 * WIDE_BN && !bias && act == 0 && ((uintptr_t)x & 15) == 0 && ((uintptr_t)w & 15) == 0) {
     const int64_t blocks = (n + WIDE_BM - 1) / WIDE_BM;
     const auto kernel = m < kWideLong ? gemm_wide_kernel<false> : gemm_wide_kernel<true>;
-    hipLaunchKernelGGL(kernel, wide_grid(blocks, m), dim3(256), 0, (hipStream_t)stream, n, m, x, w, scale, out);
+    hipLaunchKernelGGL(kernel, wide_grid(blocks, m, 1, 7), dim3(256), 0, (hipStream_t)stream, n, m, x, w, scale, out);
     FC_LAUNCH_CHECK();
     return FC_OK;
   }
@@ -1526,7 +1541,7 @@ extern "C" int fc_radial_mlp_fwd(int64_t n, int32_t n_in, const float* x, const 
   const int64_t blocks = (n + WIDE_BM - 1) / WIDE_BM;
   if (blocks > 0x7fffffff) return FC_ERR_SHAPE;
   const auto kernel = m < kWideLong ? radial_mlp_fwd_kernel<false, false> : radial_mlp_fwd_kernel<false, true>;
-  hipLaunchKernelGGL(kernel, wide_grid(blocks, m), dim3(256), 0, (hipStream_t)stream, n, (int)n_in, x, w0, s0, w1, s1,
+  hipLaunchKernelGGL(kernel, wide_grid(blocks, m, 4, 8), dim3(256), 0, (hipStream_t)stream, n, (int)n_in, x, w0, s0, w1, s1,
                      (int)m, w2, s2, out);
   FC_LAUNCH_CHECK();
   return FC_OK;
