@@ -1165,9 +1165,6 @@ static dim3 wide_grid(int64_t blocks, int m, int fixed, int pair) {
   }
   return dim3((unsigned)blocks, (unsigned)parts);
 }
-  }
-  return dim3((unsigned)blocks, (unsigned)parts);
-}
 
 template <bool LONG>
 __global__ void __launch_bounds__(256, 2) gemm_wide_kernel(int64_t n, int m, const float* __restrict__ x,
