@@ -731,22 +731,34 @@ __global__ void __launch_bounds__(256) gemm_small_kernel(GemmBatch gb) {
   g.D[off] = x;
 }
 
+// Chunks of 16 k in flight in a wave of gemm_small_kernel: those that fall to it of the batch's longest K, up to 8.
+static int small_unroll(int max_k) {
+  const int per = ((max_k + 15) / 16 + 3) / 4;
+  return per <= 1 ? 1 : per <= 2 ? 2 : per <= 4 ? 4 : 8;
+}
+
 // Whether gemm_small_kernel takes the batch: aligned groups of 4 k, and little enough work that the
 // latency of the tiled kernels, which walk all of K in one workgroup, costs more than reading every
-// operand 16 rows at a time. Work in 16 x 16 x 16 blocks: the small kernel takes 2.5 us and 1 us for
-// every 3,200, the tiled ones at least 3.4 us and 0.85 us for every 32 k. (128-wide maps, l <= 3: 32
-// nodes 7.1 -> 3.1 us, 256 nodes 7.3 us either way, 512 nodes 7.6 against 12.7; K = 512 to 896: 32 nodes 27.3
-// -> 7.1 us, 256 nodes 32 against 36.)
+// operand 16 rows at a time. Work in 16 x 16 x 16 blocks, each wave's chunks of every rank rounded up to the unroll
+// of the longest: the small kernel takes 2.5 us and 1 us for every 3,200, the tiled ones at least 3.4 us and 0.85 us for
+// every 32 k. (128-wide maps, l <= 3: 32 nodes 7.1 -> 3.1 us, 256 nodes 7.3 us either way, 512 nodes 7.6 against
+// 12.7; K = 512 to 896: 32 nodes 27.3 -> 7.1 us, 256 nodes 32 against 36; K = 320, 192, 64, 128 into 64 columns, where
+// rounding doubles to octuples the work: 100 nodes 12.5 -> 8.2 us, 300 nodes 15.4 against 13.2, 900 nodes 38 against 13.)
 static bool small_ok(const GemmBatch& gb, int n_ranks) {
-  int64_t blocks = 0;
   int max_k = 0;
   for (int l = 0; l < n_ranks; ++l) {
     const GemmRank& g = gb.r[l];
     if ((g.K & 3) || (g.a_row & 3) || (g.a_comp & 3) || ((uintptr_t)g.A & 15) || ((uintptr_t)g.P & 15) ||
         (gb.trans_b && ((uintptr_t)g.B & 15)))
       return false;
-    blocks += (int64_t)((g.M + 15) / 16) * ((g.N + 15) / 16) * ((g.K + 15) / 16);
     if (g.K > max_k) max_k = g.K;
+  }
+  const int u = small_unroll(max_k);
+  int64_t blocks = 0;
+  for (int l = 0; l < n_ranks; ++l) {
+    const GemmRank& g = gb.r[l];
+    const int64_t per = ((g.K + 15) / 16 + 3) / 4;  // chunks of a wave
+    blocks += (int64_t)((g.M + 15) / 16) * ((g.N + 15) / 16) * 4 * ((per + u - 1) / u * u);
   }
   return blocks <= 3200 + 85 * (int64_t)max_k;
 }
@@ -766,17 +778,16 @@ static int launch_small(GemmBatch gb, int n_ranks, hipStream_t s) {
   gb.n_ranks = n_ranks;
   gb.total_tiles = (int32_t)total;
   const dim3 grid((unsigned)total), block(256);
-  // U: the chunks of 16 k that fall to a wave, up to 8
-  const int per = ((max_k + 15) / 16 + 3) / 4;
   auto launch = [&](auto u) {
     constexpr int U = decltype(u)::value;
     if (gb.pair_sum) hipLaunchKernelGGL((gemm_small_kernel<false, true, U>), grid, block, 0, s, gb);
     else if (gb.trans_b) hipLaunchKernelGGL((gemm_small_kernel<false, false, U>), grid, block, 0, s, gb);
     else hipLaunchKernelGGL((gemm_small_kernel<true, false, U>), grid, block, 0, s, gb);
   };
-  if (per <= 1) launch(std::integral_constant<int, 1>{});
-  else if (per <= 2) launch(std::integral_constant<int, 2>{});
-  else if (per <= 4) launch(std::integral_constant<int, 4>{});
+  const int u = small_unroll(max_k);
+  if (u == 1) launch(std::integral_constant<int, 1>{});
+  else if (u == 2) launch(std::integral_constant<int, 2>{});
+  else if (u == 4) launch(std::integral_constant<int, 4>{});
   else launch(std::integral_constant<int, 8>{});
   FC_LAUNCH_CHECK();
   return FC_OK;
