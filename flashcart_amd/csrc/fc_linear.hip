@@ -1735,6 +1735,8 @@ struct WgradBatch {
 // its first rows are there (row cursors and addresses in scalar registers): 8 rows 5.1 -> 5.9 us, 300 rows 18.0 -> 19.0.
 // Steps that do not exist are not loaded (8 rows 6.7 us with one); loads at one place of the loop, for half the
 // code, gained nothing there and cost 3% at 25,000 rows.
+// Few outputs leave little work to the splits of many inputs: 16,384 -> 16, 40,000 rows 950 -> 1,230 us, 2,560 -> 32,
+// 25,000 nodes with l <= 2 873 -> 930; up to 900 inputs a rank it is even or faster.
 template <int TO, int TJ, bool ACT>
 __global__ void __launch_bounds__(256, 2) wgrad_kernel(WgradBatch wb) {
   constexpr int RK = 32;                    // rows per step
