@@ -605,7 +605,9 @@ def _map_bound(x, w, k):
     # enough tiles for 128-column tiles: two column tiles, the second and the last row tile partial
     (40001, 0, 0, 32, 200, [1]), (8201, 3, 3, 32, 132, [1, 2, 1, 1]),
     # the same in the input gradient (K = 96, 64): columns in two tiles, and in one that is partial
-    (40001, 0, 0, 140, 96, [1]), (8201, 3, 3, 36, 64, [1, 2, 1, 3])])
+    (40001, 0, 0, 140, 96, [1]), (8201, 3, 3, 36, 64, [1, 2, 1, 3]),
+    # ranks of different K on both sides of the line between the 16 x 16 blocks and the tiles
+    (199, 3, 3, 64, 64, [5, 3, 1, 2]), (301, 3, 3, 64, 64, [5, 3, 1, 2])])
 def test_linear_tiles(n, lin, lout, fin, fout, paths):
     """The linear maps' kernels at the edges of their tiles (rows, columns, K steps), forward with a residual and
     input gradient, against float64 with an element-wise bound."""
@@ -823,6 +825,22 @@ def test_wide_output_scaled_range(n, m):
     assert float((want / scale).abs().max()) > 3.5e38 and float(want.abs().max()) < 1e38
     bound = scale * (_map_bound(h2, w2.double(), 64) + 2.0 ** -18 * (h2.abs().amax() * w2.double().abs().sum(1)))
     assert bool(((out.double() - want).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("n,m", [(1, 2176), (2041, 2176), (12033, 1088), (21761, 704), (30001, 160), (30001, 1088),
+                                 (65536, 2176), (65537, 330)])
+def test_radial_mlp_column_parts(n, m):
+    """The radial MLP's output with its columns in one part and in several, as the numbers of row blocks and of
+    columns have it, against float64. The hidden layers' error, exp's included, is below 2^-18."""
+    ops = _ops()
+    g = torch.Generator(device=DEV).manual_seed(n + m)
+    x, w0, w1, w2 = (torch.randn(*s, device=DEV, generator=g) for s in ((n, 8), (64, 8), (64, 64), (m, 64)))
+    with torch.no_grad():
+        out = ops.radial_mlp_fwd(x, w0, 0.35, w1, 0.125, w2, 0.125)
+    h2 = O.silu(0.125 * O.silu(0.35 * x.double() @ w0.double().t()) @ w1.double().t())
+    w = w2.double()
+    bound = 0.125 * (_map_bound(h2, w, 64) + 2.0 ** -18 * (h2.abs().amax() * w.abs().sum(1)))
+    assert bool(((out.double() - 0.125 * (h2 @ w.t())).abs() <= bound).all())
 
 
 @pytest.mark.parametrize("m", [(1 << 22) - 1, 1 << 22, (1 << 23) + 5])
